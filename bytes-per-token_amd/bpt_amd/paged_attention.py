@@ -157,9 +157,12 @@ def decode_plan(
 def decode_kernel_name(
     q, k_cache, v_cache, block_table, context_lens, k_scale=None, v_scale=None, *, scale, max_context, num_splits=None
 ) -> str:
-    """The kernel the call launches: "decode_mfma_kernel" (matrix cores) or "decode_kernel" (vector)."""
+    """The kernel the call launches: "decode_mfma_kernel" (matrix cores, up to 16 rows per KV head),
+    "decode_rows_kernel" (matrix cores, more rows) or "decode_kernel" (vector)."""
     a, _, _ = _plan(q, k_cache, v_cache, block_table, context_lens, k_scale, v_scale, scale, max_context,
                     num_splits)
+    if a.rows_per_group > 16:
+        return "decode_rows_kernel"
     return "decode_mfma_kernel" if a.rows_per_group == 16 else "decode_kernel"
 
 

@@ -143,6 +143,14 @@ constexpr int kMfmaMinRows = BPT_DECODE_MFMA_MIN_ROWS;
 constexpr int kMfmaMinRowsInt8 = BPT_DECODE_MFMA_MIN_ROWS_INT8;
 constexpr int kMfmaRows = 16;
 constexpr int kMfmaChunk = 32;
+// Many-row attention (decode_rows.h): chunks of kRowsChunk tokens, tiles of 32, 64 or 128 rows.
+constexpr int kRowsChunk = 128;
+constexpr int rows_tile(int rows) { return rows <= 32 ? 32 : rows <= 64 ? 64 : 128; }
+constexpr int rows_groups_per_cu(int tile) { return tile == 32 ? 2 : 1; }
+constexpr int kRowsMinChunks = 1;
+constexpr int kRowsPieceCost = 2;
+// Largest tile line the kernel takes, in tiles and sequences of one KV head: 4-byte entries in LDS.
+constexpr int64_t kRowsMaxLine = 4096;
 // Waves per SIMD the matrix-core decode kernel is compiled for (its register budget: 512 / this).
 constexpr int kMfmaWavesPerSimd = BPT_DECODE_MFMA_WAVES_PER_SIMD;
 
@@ -330,6 +338,9 @@ hipError_t launch_decode(const DecodeParams& p, int kv_dtype, int scale_kind, in
                          const LaunchEvents& ev = {});
 hipError_t launch_decode_mfma(const DecodeParams& p, int kv_dtype, int scale_kind, hipStream_t stream,
                               const LaunchEvents& ev = {});
+hipError_t launch_rows_32(const DecodeParams& p, int kv_dtype, int scale_kind, hipStream_t stream, const LaunchEvents& ev);
+hipError_t launch_rows_64(const DecodeParams& p, int kv_dtype, int scale_kind, hipStream_t stream, const LaunchEvents& ev);
+hipError_t launch_rows_128(const DecodeParams& p, int kv_dtype, int scale_kind, hipStream_t stream, const LaunchEvents& ev);
 hipError_t launch_kivi(const KiviParams& p, int fmt, hipStream_t stream);
 // Any even head dim up to 256 and float32 bits-16 caches: one workgroup per (sequence, KV head, split).
 hipError_t launch_kivi_any(const KiviParams& p, int fmt, hipStream_t stream);

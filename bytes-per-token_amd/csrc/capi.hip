@@ -45,6 +45,7 @@ bool aligned_to(const void* p, int64_t stride_b, int64_t stride_q, int64_t strid
 
 struct Plan {
   bool mfma;  // the matrix-core kernel (all rows of a KV head in one 16-row group)
+  bool tiles;  // the many-row matrix-core kernel (decode_rows.h): tiles of rows_per_group rows
   int rows, rows_per_group, n_rg, HR, chunk, grid, len_cap;
   int64_t per_forced;
   int equal_grid;  // workgroups that take equal partitions when all lengths are equal (0: none)
@@ -59,7 +60,18 @@ std::mutex g_tuning_mutex;
 
 size_t align256(size_t x) { return (x + 255) & ~(size_t)255; }
 
-int make_plan(const bpt_decode_args* a, Plan* pl) {
+// Whether a call with more than 16 rows per KV head takes the many-row kernel: a bf16 or f16 q (an f32 q keeps the
+// vector kernel's float32 products), 16 token strides of a page within 32 bits, and a tile line that fits its LDS.
+bool takes_tiles(const bpt_decode_args* a, int rows, int tile) {
+  if (rows <= bpt::kMfmaRows || a->q_dtype == BPT_F_F32) return false;
+  const int64_t stok = a->kv_stride_token * (a->kv_dtype == BPT_KV_BF16 ? 2 : 1);
+  if (stok < 0 || 16 * stok >= (int64_t(1) << 31)) return false;
+  const int64_t tiles = ((int64_t)rows + tile - 1) / tile;
+  return (int64_t)a->batch * (tiles + 1) <= bpt::kRowsMaxLine;
+}
+
+// tiles_ok: whether the many-row kernel may be chosen.
+int make_plan(const bpt_decode_args* a, Plan* pl, bool tiles_ok = true) {
   const char* fn = "bpt_decode_plan";
   if (!a) return fail(BPT_ERR_INVALID_ARGUMENT, "%s: args is NULL", fn);
   if (a->struct_size != sizeof(bpt_decode_args))
@@ -98,12 +110,14 @@ int make_plan(const bpt_decode_args* a, Plan* pl) {
   // from 5 rows on (with fewer, the vector kernel reads each page once too and its INT8 decode is cheaper).
   pl->mfma = pl->rows <= bpt::kMfmaRows && ((a->kv_dtype == BPT_KV_FP8_E4M3FN && pl->rows >= bpt::kMfmaMinRows) ||
                                             (a->kv_dtype == BPT_KV_INT8 && pl->rows >= bpt::kMfmaMinRowsInt8));
-  pl->rows_per_group = pl->mfma ? bpt::kMfmaRows : (pl->rows <= 1 ? 1 : (pl->rows <= 2 ? 2 : 4));
+  const int tile = bpt::rows_tile(pl->rows);
+  pl->tiles = tiles_ok && takes_tiles(a, pl->rows, tile);
+  pl->rows_per_group = pl->tiles ? tile : pl->mfma ? bpt::kMfmaRows : (pl->rows <= 1 ? 1 : (pl->rows <= 2 ? 2 : 4));
   pl->n_rg = (pl->rows + pl->rows_per_group - 1) / pl->rows_per_group;
   const int64_t hr = (int64_t)a->num_kv_heads * pl->n_rg;
   if (hr > (1 << 20)) return fail(BPT_ERR_INVALID_ARGUMENT, "%s: too many KV heads x row groups", fn);
   pl->HR = (int)hr;
-  pl->chunk = pl->mfma ? bpt::kMfmaChunk : bpt::decode_chunk_tokens(a->kv_dtype, pl->rows_per_group);
+  pl->chunk = pl->tiles ? bpt::kRowsChunk : pl->mfma ? bpt::kMfmaChunk : bpt::decode_chunk_tokens(a->kv_dtype, pl->rows_per_group);
   const int64_t table_cap = (int64_t)a->max_blocks_per_seq * a->page_size;
   pl->len_cap = (int)(a->max_context < table_cap ? a->max_context : table_cap);
   const int64_t max_nb = (pl->len_cap + pl->chunk - 1) / pl->chunk;
@@ -125,6 +139,7 @@ int make_plan(const bpt_decode_args* a, Plan* pl) {
   const bool pair = pl->waves == bpt::kMfmaPairWaves;
   const int groups_per_cu =
       tune.groups_per_cu > 0 ? tune.groups_per_cu
+      : pl->tiles ? bpt::rows_groups_per_cu(tile)
       : pair ? bpt::kMfmaPairGroupsPerCu
       : pl->mfma ? bpt::mfma_groups_per_cu(pl->rows)
                  : bpt::decode_groups_per_cu(a->kv_dtype == BPT_KV_INT8, pl->rows_per_group,
@@ -148,10 +163,11 @@ int make_plan(const bpt_decode_args* a, Plan* pl) {
     pl->per_forced = 0;
     int64_t grid = (int64_t)bpt::kComputeUnits * groups_per_cu;
     const int64_t min_chunks = tune.min_chunks > 0 ? tune.min_chunks
+                               : pl->tiles ? bpt::kRowsMinChunks
                                : bpt::decode_min_chunks(pl->mfma, pl->rows, a->kv_dtype == BPT_KV_INT8, bound_c);
     const int64_t fill = (bound_c + min_chunks - 1) / min_chunks;
     if (fill < grid) grid = fill;
-    if (!pl->mfma && bound_c > 0 &&
+    if (!pl->mfma && !pl->tiles && bound_c > 0 &&
         ((a->kv_dtype == BPT_KV_BF16 && bound_c <= bpt::kAlignedMaxChunksBf16) ||
          (a->kv_dtype == BPT_KV_INT8 && bound_c <= bpt::kAlignedMaxChunksInt8))) {
       // About 4 sqrt(chunks) workgroups (at most 512) take equal partitions of a power-of-two number of
@@ -179,10 +195,12 @@ int make_plan(const bpt_decode_args* a, Plan* pl) {
   // for the merges (measured on the matrix-core kernel at 512 / 2943 tokens: 11.1 -> 9.5, 12.9 -> 12.0 us).
   pl->piece_cost = pl->per_forced > 0 ? 0
                    : tune.piece_cost >= 0 ? tune.piece_cost
+                   : pl->tiles ? bpt::kRowsPieceCost
                    : a->batch == 1 ? 0
                    : pair ? bpt::kMfmaPairPieceCost
                    : (pl->mfma && pl->rows >= bpt::kManyRows ? bpt::kManyRowPieceCost : bpt::kDecodePieceCost);
-  const size_t slots = (size_t)a->batch * pl->HR + pl->grid;
+  // The many-row kernel's workgroups hold at most two partials each: the first and the last piece of their range.
+  const size_t slots = pl->tiles ? 2 * (size_t)pl->grid : (size_t)a->batch * pl->HR + pl->grid;
   pl->ws_out_floats = slots * pl->rows_per_group * a->head_dim;
   pl->ws_lse_floats = slots * pl->rows_per_group;
   pl->workspace = align256((pl->ws_out_floats + pl->ws_lse_floats) * sizeof(float));
@@ -437,8 +455,11 @@ int paged_decode(const bpt_decode_args* a, void* stream, const bpt::LaunchEvents
     p.w_sq = fuse->s_sq;
     p.w_i64 = fuse->slot_i64;
   }
-  hipError_t e = pl.mfma ? bpt::launch_decode_mfma(p, a->kv_dtype, a->scale_kind, (hipStream_t)stream, ev)
-                         : bpt::launch_decode(p, a->kv_dtype, a->scale_kind, pl.rows_per_group, (hipStream_t)stream, ev);
+  hipError_t e = pl.tiles  ? (pl.rows_per_group == 32   ? bpt::launch_rows_32
+                              : pl.rows_per_group == 64 ? bpt::launch_rows_64
+                                                        : bpt::launch_rows_128)(p, a->kv_dtype, a->scale_kind, (hipStream_t)stream, ev)
+                 : pl.mfma ? bpt::launch_decode_mfma(p, a->kv_dtype, a->scale_kind, (hipStream_t)stream, ev)
+                           : bpt::launch_decode(p, a->kv_dtype, a->scale_kind, pl.rows_per_group, (hipStream_t)stream, ev);
   if (e != hipSuccess) return hip_fail(fn, e);
   return BPT_OK;
 }
@@ -473,7 +494,7 @@ int bpt_set_tuning(const bpt_tuning* t) {
 // only form passed to kernels.
 namespace {
 
-constexpr size_t kScratchWorkspace = (size_t)30 << 20;
+constexpr size_t kScratchWorkspace = (size_t)34 << 20;  // the many-row kernel's largest: 512 slots of 128 rows
 constexpr size_t kScratchCounters = (size_t)2 << 20;
 constexpr int kMaxDevices = 64;
 
@@ -966,7 +987,7 @@ int bpt_page_read_probe(const bpt_decode_args* a, float* partial_sums, int64_t* 
                         void* start_event, void* stop_event) {
   const char* fn = "bpt_page_read_probe";
   Plan pl;
-  int rc = make_plan(a, &pl);
+  int rc = make_plan(a, &pl, false);  // the probe reads in the other kernels' order
   if (rc) return rc;
   const int64_t g = a->batch > 0 ? pl.grid : 0;  // the decode's workgroups
   if (num_groups) *num_groups = g;

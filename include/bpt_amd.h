@@ -111,7 +111,8 @@ typedef struct {
   int32_t chunk_tokens; /* out of bpt_decode_plan: tokens one wave streams per step */
   int32_t grid_groups;  /* out of bpt_decode_plan: workgroups launched */
   int32_t rows_per_group; /* out of bpt_decode_plan: query rows computed together per KV head; 16 = the
-                             matrix-core kernel (FP8 caches, 2..16 rows), 1/2/4 = the vector kernel */
+                             matrix-core kernel (FP8 caches, 2..16 rows; INT8, 5..16), 32/64/128 = the many-row
+                             matrix-core kernel (more than 16 rows), 1/2/4 = the vector kernel */
   float sm_scale;
 
   const void* q;
@@ -368,7 +369,7 @@ int bpt_decode_plan(bpt_decode_args* args, size_t* workspace_bytes, size_t* coun
 int bpt_paged_decode(const bpt_decode_args* args, void* stream);
 
 /* bpt_paged_decode with no caller workspace: the split-K partials and arrival counters live in a device-
- * resident array of the library (30 MiB of partials and 2 MiB of counters on each GPU it runs on, held until the
+ * resident array of the library (34 MiB of partials and 2 MiB of counters on each GPU it runs on, held until the
  * process ends), so the call allocates nothing: for callers that cannot allocate (code under HIP graph
  * capture, tight serving loops, harnesses that forbid hipMalloc). No counterpart in the reference. The
  * workspace and counters fields of args are ignored; a call whose bpt_decode_plan sizes exceed the array's

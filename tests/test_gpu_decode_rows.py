@@ -1,0 +1,72 @@
+"""GPU: the many-row kernel (more than 16 query rows per KV head, decode_rows.h) against the oracle.
+
+Sizes sit at the edges of its tiles (32, 64 and 128 rows), chunks (128 tokens) and pages. bf16 results at the decode
+tolerance; float32 results within 2^-14 of the largest output: the value weights carry at least 22 bits, so what is
+left is the float32 rounding of scores up to 2^7 base-2 units (2^-18 each, on both sides: a weight off by up to
+2^-17 ln 2 in the kernel and in the oracle, times the few that accumulate).
+"""
+
+import numpy as np
+import pytest
+import torch
+
+from test_gpu_decode import DEV, check, make_case, run_case
+
+pytestmark = pytest.mark.gpu
+
+FORMATS = [("fp8", "head"), ("int8", "token"), ("bf16", None), ("int8", "head"), ("fp8", "token")]
+
+
+@pytest.mark.parametrize("fmt,scales", FORMATS)
+@pytest.mark.parametrize("nq,hq,hkv", [(17, 4, 4), (16, 4, 2), (11, 6, 2), (32, 4, 2), (13, 10, 2), (64, 2, 1), (43, 3, 1), (150, 4, 2)])
+def test_rows_at_tile_edges(fmt, scales, nq, hq, hkv):
+    c = make_case(fmt, [517, 0, nq, 128, 129, 1, 260], hq=hq, hkv=hkv, nq=nq, scales=scales, seed=nq)
+    got, want = run_case(c)
+    check(got, want, f"{fmt}/{scales} {nq} queries, {hq}/{hkv} heads")
+    assert got[1].float().abs().sum().item() == 0  # no tokens: zeros
+
+
+@pytest.mark.parametrize("fmt,scales", FORMATS)
+@pytest.mark.parametrize("page", [1, 2, 8, 16, 128])
+@pytest.mark.parametrize("q_dtype", [torch.bfloat16, torch.float16])
+def test_rows_page_sizes_and_q_dtypes(fmt, scales, page, q_dtype):
+    c = make_case(fmt, [300, 77], hq=8, hkv=2, nq=9, page=page, scales=scales, seed=page, table_dtype=torch.int64)
+    got, want = run_case(c, q=c["q"].to(q_dtype), out_dtype=q_dtype)
+    check(got, want, f"{fmt}/{scales} page {page} {q_dtype}")
+
+
+@pytest.mark.parametrize("num_splits", [1, 3, 1000])
+@pytest.mark.parametrize("nq", [10, 20, 40])
+def test_rows_forced_splits(num_splits, nq):
+    c = make_case("fp8", [2000, 131, 40], hq=8, hkv=2, nq=nq, seed=num_splits)
+    got, want = run_case(c, num_splits=num_splits)
+    check(got, want, f"{nq} queries, {num_splits} splits")
+
+
+@pytest.mark.parametrize("fmt,scales", FORMATS)
+@pytest.mark.parametrize("nq,q_dtype", [(10, torch.bfloat16), (20, torch.float16), (40, torch.bfloat16)])
+def test_rows_long_context_in_float32(fmt, scales, nq, q_dtype):
+    c = make_case(fmt, [9000, 700], hq=8, hkv=2, nq=nq, scales=scales, seed=nq, head_major=True)
+    got, want = run_case(c, q=c["q"].to(q_dtype), out_dtype=torch.float32)
+    err = np.abs(got.cpu().numpy() - want).max()
+    assert err <= 2.0**-14 * np.abs(want).max(), f"{fmt}/{scales}: {err:.3e}"
+
+
+def test_rows_negative_scale_and_lse_and_repeats():
+    from bpt_amd import paged_decode_attention
+    from oracle import attention
+    from test_gpu_decode import np_codes
+
+    c = make_case("fp8", [900, 33], hq=8, hkv=2, nq=12, seed=5)
+    lse = torch.empty((2, 12, 8), device=DEV)
+    args = (c["q"], c["k"], c["v"], c["table"], c["lens"], c["ks"], c["vs"])
+    got = paged_decode_attention(*args, scale=-0.05, max_context=900, lse=lse, out_dtype=torch.float32)
+    again = paged_decode_attention(*args, scale=-0.05, max_context=900, out_dtype=torch.float32)
+    want, want_lse = attention.paged_decode(
+        c["q"].float().cpu().numpy(), np_codes(c["k"], "fp8"), np_codes(c["v"], "fp8"), c["table"].cpu().numpy(),
+        c["lens"].cpu().numpy(), c["ks"].cpu().numpy(), c["vs"].cpu().numpy(), "fp8", -0.05)
+    assert torch.equal(got, again)
+    assert np.abs(got.cpu().numpy() - want).max() <= 2.0**-14 * np.abs(want).max()
+    seen = np.isfinite(want_lse)
+    assert np.array_equal(np.isfinite(lse.cpu().numpy()), seen)
+    assert np.abs(lse.cpu().numpy() - want_lse)[seen].max() < 1e-4
