@@ -620,6 +620,13 @@ __device__ __forceinline__ void load_q_fold(const KiviParams& p, int b, int h, i
   }
 }
 
+// This wave's LDS writes become visible to its own lanes' later reads.
+__device__ __forceinline__ void wave_sync() {
+  __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+  __builtin_amdgcn_wave_barrier();
+  __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+}
+
 __device__ __forceinline__ int64_t out_index(const KiviParams& p, int b, int hq, int j) {
   return (int64_t)b * p.o_sb + (int64_t)hq * p.o_sh + (int64_t)j * p.o_ss;
 }
@@ -628,78 +635,159 @@ __device__ __forceinline__ int64_t lse_index(const KiviParams& p, int b, int hq,
   return (int64_t)b * p.l_sb + (int64_t)hq * p.l_sh + (int64_t)j * p.l_ss;
 }
 
-// Splits past a row's length: out 0, lse -inf (workgroups take the rows round-robin).
-// The attention state of the full-precision tail for the G query heads of (b, h), in the wave states' form
-// (base 2, reference point m, bias kBias): s_tm[r] = m_r = max_t s_rt, s_tl[r] = sum_t 2^(s_rt - m_r + kBias),
-// s_to[r D + ch] = sum_t 2^(s_rt - m_r + kBias) v_t[ch], where s_rt = sm_scale log2(e) q_r . k_t over the
-// tail_len tokens (fastserve integration/kv_cache.py:179-182: partial_attention over the tail, in float32).
-// s_tp: G x kKiviMaxTail floats of scratch. The whole workgroup calls it; it ends with a barrier.
-template <int NT>
-__device__ __forceinline__ void tail_state(const KiviParams& p, int b, int h, float* s_tp, float* s_tm, float* s_tl,
-                                           float* s_to) {
-  constexpr int D = kHeadDim;
-  const int T = p.tail_len, G = p.G;
-  const int64_t kv0 = (int64_t)b * p.tk_sb + (int64_t)h * p.tk_sh;
-  for (int i = threadIdx.x; i < G * T; i += NT) {
-    const int r = i / T, t = i - r * T;
-    const int64_t qo = (int64_t)b * p.q_sb + (int64_t)(h * G + r) * p.q_sh;
-    const int64_t ko = kv0 + (int64_t)t * p.tk_st;
-    float acc = 0.0f;
-#pragma unroll 8
-    for (int c = 0; c < D; ++c) acc = fmaf(load_float(p.q, qo + c, p.q_dtype), load_float(p.tk, ko + c, p.tail_dtype), acc);
-    s_tp[r * kKiviMaxTail + t] = acc * p.qscale;
-  }
-  __syncthreads();
-  for (int r = threadIdx.x; r < G; r += NT) {
-    float m = kNegInf;
-    for (int t = 0; t < T; ++t) m = fmaxf(m, s_tp[r * kKiviMaxTail + t]);
-    float l = 0.0f;
-    for (int t = 0; t < T; ++t) {
-      const float w = fast_exp2(s_tp[r * kKiviMaxTail + t] - m + kBias);
-      s_tp[r * kKiviMaxTail + t] = w;
-      l += w;
+// This wave's share of the full-precision tail for the G query heads of (b, h): tokens 16 i + 4 wave + lane / 16,
+// folded in float32 into a wave state (base 2, reference point m, bias kBias) in LDS: s_m[r] = m_r, its largest
+// score (-inf without tokens), s_l[r] = sum_t 2^(s_rt - m_r + kBias), s_o[r][ch] = sum_t 2^(s_rt - m_r + kBias)
+// v_t[ch], where s_rt = sm_scale log2(e) q_r . k_t (fastserve integration/kv_cache.py:179-182: partial_attention
+// over the tail). s_o holds the q rows on entry (unscaled, stored by this wave).
+//
+// What bounds it is latency, so every key and value of the wave is requested at once (16 lanes of 8 channels to
+// a token, one 16-byte load each for aligned 16-bit tails) and the call comes before the piece's chunk loop,
+// whose first chunks are in flight meanwhile. (One thread per score and per output channel, after the loop: 16
+// serial rounds of strided loads. 16 sequences, 8 KV heads, 2 rows, 2048 4-bit tokens and 17 in the tail: 54.0 us,
+// now 23.4, and 18.2 without a tail; 8-bit codes with 31 in the tail 25.7, without 20.9.)
+template <int RP>
+__device__ __forceinline__ void tail_state(const KiviParams& p, int b, int h, int wave, int lane, float* s_m, float* s_l,
+                                           float (*s_o)[kHeadDim + 1]) {
+  constexpr int NI = kKiviMaxTail / 16;
+  const int T = p.tail_len;
+  const int part = lane & 15;
+  const int64_t at = (int64_t)b * p.tk_sb + (int64_t)h * p.tk_sh + 8 * part;
+  const int eb = p.tail_dtype == kFF32 ? 4 : 2;
+  const bool wide = eb == 2 && (((uintptr_t)p.tk | (uintptr_t)p.tv) & 15) == 0 && ((p.tk_sb | p.tk_sh | p.tk_st) & 7) == 0;
+  float kf[NI][8], vf[NI][8];
+  if (wide) {
+    u32x4 kw[NI], vw[NI];
+#pragma unroll
+    for (int i = 0; i < NI; ++i) {
+      const int t = 16 * i + 4 * wave + (lane >> 4);
+      kw[i] = u32x4{0u, 0u, 0u, 0u};
+      vw[i] = u32x4{0u, 0u, 0u, 0u};
+      if (t < T) {
+        kw[i] = *(const u32x4*)((const uint16_t*)p.tk + at + (int64_t)t * p.tk_st);
+        vw[i] = *(const u32x4*)((const uint16_t*)p.tv + at + (int64_t)t * p.tk_st);
+      }
     }
-    s_tm[r] = m;
-    s_tl[r] = l;
+    const bool bf = p.tail_dtype == kFBf16;
+    auto lo = [&](uint32_t w) { return bf ? __uint_as_float(w << 16) : (float)__builtin_bit_cast(_Float16, (uint16_t)w); };
+    auto hi = [&](uint32_t w) {
+      return bf ? __uint_as_float(w & 0xffff0000u) : (float)__builtin_bit_cast(_Float16, (uint16_t)(w >> 16));
+    };
+#pragma unroll
+    for (int i = 0; i < NI; ++i) {
+#pragma unroll
+      for (int j = 0; j < 4; ++j) {
+        kf[i][2 * j] = lo(kw[i][j]);
+        kf[i][2 * j + 1] = hi(kw[i][j]);
+        vf[i][2 * j] = lo(vw[i][j]);
+        vf[i][2 * j + 1] = hi(vw[i][j]);
+      }
+    }
+  } else {
+#pragma unroll
+    for (int i = 0; i < NI; ++i) {
+      const int t = 16 * i + 4 * wave + (lane >> 4);
+#pragma unroll
+      for (int j = 0; j < 8; ++j) kf[i][j] = vf[i][j] = 0.0f;
+      if (t < T) {
+        const int64_t o = at + (int64_t)t * p.tk_st;
+#pragma unroll
+        for (int j = 0; j < 8; ++j) {
+          kf[i][j] = load_float(p.tk, o + j, p.tail_dtype);
+          vf[i][j] = load_float(p.tv, o + j, p.tail_dtype);
+        }
+      }
+    }
   }
-  __syncthreads();
-  for (int i = threadIdx.x; i < G * D; i += NT) {
-    const int r = i / D, ch = i - r * D;
-    float o = 0.0f;
-    for (int t = 0; t < T; ++t) o = fmaf(s_tp[r * kKiviMaxTail + t], load_float(p.tv, kv0 + (int64_t)t * p.tk_st + ch, p.tail_dtype), o);
-    s_to[r * D + ch] = o;
+  for (int r = 0; r < p.G; ++r) {
+    float q[8], s[NI];
+#pragma unroll
+    for (int j = 0; j < 8; ++j) q[j] = s_o[r][8 * part + j];
+    float m = kNegInf;
+#pragma unroll
+    for (int i = 0; i < NI; ++i) {
+      float a0 = 0.0f, a1 = 0.0f;
+#pragma unroll
+      for (int j = 0; j < 8; j += 2) {
+        a0 = fmaf(q[j], kf[i][j], a0);
+        a1 = fmaf(q[j + 1], kf[i][j + 1], a1);
+      }
+      const float x = group_sum<16>(a0 + a1) * p.qscale;
+      s[i] = 16 * i + 4 * wave + (lane >> 4) < T ? x : kNegInf;
+      m = fmaxf(m, s[i]);
+    }
+    m = max_xor<32>(max_xor<16>(m));
+    const float base = (m == kNegInf ? 0.0f : m) - kBias;
+    float l = 0.0f, o[8] = {0.0f, 0.0f, 0.0f, 0.0f, 0.0f, 0.0f, 0.0f, 0.0f};
+#pragma unroll
+    for (int i = 0; i < NI; ++i) {
+      const float w = fast_exp2(s[i] - base);
+      l += w;
+#pragma unroll
+      for (int j = 0; j < 8; ++j) o[j] = fmaf(w, vf[i][j], o[j]);
+    }
+    l = sum_xor<32>(sum_xor<16>(l));
+#pragma unroll
+    for (int j = 0; j < 8; ++j) o[j] = sum_xor<32>(sum_xor<16>(o[j]));
+    if (lane < 16) {
+#pragma unroll
+      for (int j = 0; j < 8; ++j) s_o[r][8 * part + j] = o[j];
+      if (lane == 0) {
+        s_m[r] = m;
+        s_l[r] = l;
+      }
+    }
   }
-  __syncthreads();
 }
 
-template <int NT, bool TAIL>
-__device__ __forceinline__ void zero_empty_splits(const KiviParams& p, const int* s_prefix, float* s_tp, float* s_tm,
-                                                  float* s_tl, float* s_to) {
-  constexpr int D = kHeadDim;
-  for (int b = blockIdx.x; b < p.B; b += gridDim.x) {
-    const int nb = s_prefix[b + 1] - s_prefix[b];
-    if (TAIL && nb == 0) {  // no codes: the result is the tail's attention alone (one split)
-      for (int h = 0; h < p.Hkv; ++h) {
-        tail_state<NT>(p, b, h, s_tp, s_tm, s_tl, s_to);
-        for (int i = threadIdx.x; i < p.G * D; i += NT) {
-          const int r = i / D, ch = i - r * D;
-          const int hq = h * p.G + r;
-          p.out[out_index(p, b, hq, 0) + ch] = s_to[r * D + ch] / s_tl[r];
-          if (ch == 0) p.lse[lse_index(p, b, hq, 0)] = (s_tm[r] - kBias + __log2f(s_tl[r])) * kLn2;
-        }
-        __syncthreads();  // the tail buffers are rewritten by the next head
+// Splits past a row's length: out 0, lse -inf (workgroups take the rows round-robin). With a tail (one split), a
+// row without codes gets the tail's attention alone.
+template <int NW, int RP, bool TAIL>
+__device__ __forceinline__ void zero_empty_splits(const KiviParams& p, const int* s_prefix, float (*s_m)[RP], float (*s_l)[RP],
+                                                  float (*s_o)[RP][kHeadDim + 1]) {
+  constexpr int D = kHeadDim, NT = NW * 64;
+  if constexpr (TAIL) {
+    const int lane = threadIdx.x & 63, wave = sread(threadIdx.x >> 6);
+    for (int bh = blockIdx.x; bh < p.B * p.Hkv; bh += gridDim.x) {
+      const int b = bh / p.Hkv, h = bh - b * p.Hkv;
+      if (s_prefix[b + 1] != s_prefix[b]) continue;
+      for (int i = lane; i < p.G * D; i += 64) {
+        const int64_t qo = (int64_t)b * p.q_sb + (int64_t)(h * p.G + i / D) * p.q_sh;
+        s_o[wave][i / D][i % D] = load_float(p.q, qo + i % D, p.q_dtype);
       }
-      continue;
+      wave_sync();
+      tail_state<RP>(p, b, h, wave, lane, s_m[wave], s_l[wave], s_o[wave]);
+      __syncthreads();
+      for (int i = threadIdx.x; i < p.G * D; i += NT) {
+        const int r = i / D, ch = i - r * D;
+        const int hq = h * p.G + r;
+        float M = kNegInf, L = 0.0f, A = 0.0f;
+#pragma unroll
+        for (int w = 0; w < NW; ++w) M = fmaxf(M, s_m[w][r]);
+        const float mu = M == kNegInf ? 0.0f : M;
+#pragma unroll
+        for (int w = 0; w < NW; ++w) {
+          const float e = fast_exp2(s_m[w][r] - mu);
+          L = fmaf(s_l[w][r], e, L);
+          A = fmaf(s_o[w][r][ch], e, A);
+        }
+        p.out[out_index(p, b, hq, 0) + ch] = A / L;
+        if (ch == 0) p.lse[lse_index(p, b, hq, 0)] = (M - kBias + __log2f(L)) * kLn2;
+      }
+      __syncthreads();  // the next head's states go to the same buffers
     }
-    const int active = (nb + p.cps - 1) / p.cps;
-    const int per_head = (p.S - active) * D;
-    for (int i = threadIdx.x; i < p.Hq * per_head; i += NT) {
-      const int hq = i / per_head;
-      const int r = i - hq * per_head;
-      const int j = active + r / D;
-      const int ch = r % D;
-      p.out[out_index(p, b, hq, j) + ch] = 0.0f;
-      if (ch == 0) p.lse[lse_index(p, b, hq, j)] = kNegInf;
+  } else {
+    for (int b = blockIdx.x; b < p.B; b += gridDim.x) {
+      const int active = (s_prefix[b + 1] - s_prefix[b] + p.cps - 1) / p.cps;
+      const int per_head = (p.S - active) * D;
+      for (int i = threadIdx.x; i < p.Hq * per_head; i += NT) {
+        const int hq = i / per_head;
+        const int r = i - hq * per_head;
+        const int j = active + r / D;
+        const int ch = r % D;
+        p.out[out_index(p, b, hq, j) + ch] = 0.0f;
+        if (ch == 0) p.lse[lse_index(p, b, hq, j)] = kNegInf;
+      }
     }
   }
 }
@@ -782,11 +870,6 @@ __global__ __launch_bounds__(kDecodeWaves * 64, 2) void kivi_decode_kernel(const
   __shared__ float s_m[NW][RP];
   __shared__ float s_l[NW][RP];
   __shared__ float s_o[NW][RP][D + 1];  // rows padded by one word: a merge store's rows land on distinct banks
-  __shared__ float s_tm[RP], s_tl[RP];  // the tail's state (tail_state); its scratch and sums reuse the fold buffers
-  static_assert(sizeof(s_qh) >= RP * kKiviMaxTail * sizeof(float) && sizeof(s_ql) >= RP * D * sizeof(float),
-                "the fold buffers hold the tail's scratch");
-  float* const s_tp = (float*)&s_qh[0][0][0];
-  float* const s_to = (float*)&s_ql[0][0][0];
 
   const int tid = threadIdx.x;
   const int lane = tid & 63;
@@ -797,7 +880,7 @@ __global__ __launch_bounds__(kDecodeWaves * 64, 2) void kivi_decode_kernel(const
   const int G = p.G;
 
   build_segment_line<NW, kChunk>(p, s_prefix, s_len, s_wsum);
-  zero_empty_splits<NT, TAIL>(p, s_prefix, s_tp, s_tm, s_tl, s_to);
+  zero_empty_splits<NW, RP, TAIL>(p, s_prefix, s_m, s_l, s_o);
 
   // ---- this workgroup's range of chunks on the line of (sequence, KV head) segments ---------------------
   const int C = HR * s_prefix[B];  // < 2^31, checked on the host
@@ -874,6 +957,17 @@ __global__ __launch_bounds__(kDecodeWaves * 64, 2) void kivi_decode_kernel(const
     const int k_end = piece_end(k, c);
     const int seg_c0 = HR * s_prefix[b] + h * nb;
     const int split_end = min((j_cur + 1) * p.cps, nb);
+
+    // The piece that starts the segment also holds the tail's tokens (one split: the tail goes with it). Its
+    // waves' shares wait in s_m, s_l and s_o until the chunks are done.
+    const bool with_tail = TAIL && k_first == 0;
+    if (with_tail) {
+#pragma unroll
+      for (int c1 = 0; c1 < CPL; ++c1) s_o[wave][lane / LPR][(lane % LPR) * CPL + c1] = qf[c1];
+      wave_sync();
+      tail_state<RP>(p, b, h, wave, lane, s_m[wave], s_l[wave], s_o[wave]);
+      wave_sync();
+    }
 
     float m = kNegInf, l = 0.0f;
     f32x4 o[8], oz = {0.0f, 0.0f, 0.0f, 0.0f};
@@ -972,6 +1066,22 @@ __global__ __launch_bounds__(kDecodeWaves * 64, 2) void kivi_decode_kernel(const
     // stored for the workgroup merge.
     if constexpr (F::template kZeroFold<CPL>) value_zero_out<FMT>(kq, oz, o);
     l = sum_xor<32>(sum_xor<16>(l));
+    if (with_tail) {  // + this wave's share of the tail
+      const int r = n < G ? n : 0;
+      const float tm = s_m[wave][r];
+      const float mn = fmaxf(m, tm);
+      const float mu0 = mn == kNegInf ? 0.0f : mn;
+      const float e = l > 0.0f ? fast_exp2(m - mu0) : 0.0f, te = fast_exp2(tm - mu0);
+      l = l * e + s_l[wave][r] * te;
+#pragma unroll
+      for (int mu = 0; mu < 8; ++mu) {
+#pragma unroll
+        for (int i = 0; i < 4; ++i)
+          o[mu][i] = (e > 0.0f ? o[mu][i] * e : 0.0f) + s_o[wave][r][out_channel<FMT>(kq, i, mu)] * te;
+      }
+      m = mn;
+      wave_sync();
+    }
     if (n < RP) {
       if (kq == 0) {
         s_m[wave][n] = m;
@@ -984,9 +1094,6 @@ __global__ __launch_bounds__(kDecodeWaves * 64, 2) void kivi_decode_kernel(const
       }
     }
     __syncthreads();
-    // The piece that starts the segment also holds the tail's tokens (one split: the tail goes with it).
-    const bool with_tail = TAIL && k_first == 0;
-    if (with_tail) tail_state<NT>(p, b_cur, h_cur, s_tp, s_tm, s_tl, s_to);
 
     // ---- merge the waves; write the split's result, or this piece's partial ---------------------------
     const int seg = (b_cur * HR + h_cur) * p.S + j_cur;
@@ -1002,20 +1109,15 @@ __global__ __launch_bounds__(kDecodeWaves * 64, 2) void kivi_decode_kernel(const
       float M = kNegInf;
 #pragma unroll
       for (int w = 0; w < NW; ++w) M = fmaxf(M, s_m[w][r]);
-      if (with_tail) M = fmaxf(M, s_tm[r]);
       const float mu = M == kNegInf ? 0.0f : M;
       float L = 0.0f, A = 0.0f;
 #pragma unroll
       for (int w = 0; w < NW; ++w) {
         const float lw = s_l[w][r];
-        const float e = lw > 0.0f ? fast_exp2(s_m[w][r] - mu) : 0.0f;
+        const bool in = TAIL ? lw != 0.0f : lw > 0.0f;  // a NaN tail makes the piece empty, as one state would
+        const float e = in ? fast_exp2(s_m[w][r] - mu) : 0.0f;
         L += lw * e;
-        A += lw > 0.0f ? s_o[w][r][ch] * e : 0.0f;
-      }
-      if (with_tail) {
-        const float e = fast_exp2(s_tm[r] - mu);
-        L += s_tl[r] * e;
-        A += s_to[r * D + ch] * e;
+        A += in ? s_o[w][r][ch] * e : 0.0f;
       }
       const float out = L > 0.0f ? A / L : 0.0f;
       const float lse2 = L > 0.0f ? M - kBias + __log2f(L) : kNegInf;

@@ -79,6 +79,30 @@ def test_tail_dtypes_and_head_ratios(tail_dtype, q_heads):
     close(got, want_step(qn, ref, lengths, tkn, tvn, 0.088), f"{tail_dtype} G {q_heads // 8}")
 
 
+@pytest.mark.parametrize("layout", ["whole rows", "odd offset", "odd token stride"])
+@pytest.mark.parametrize("tail_dtype", [torch.bfloat16, torch.float16, torch.float32])
+@pytest.mark.parametrize("q_heads, tail_len", [(8, 4), (16, 5), (64, 17), (128, 64)])
+def test_tail_splits_over_waves_and_loads(q_heads, tail_len, tail_dtype, layout):
+    """Each wave takes 4 of every 16 tail tokens (with 4 tokens three waves have none) and 16-bit rows on 16 bytes
+    are read whole, others by element; 1 .. 16 query heads per KV head; a row of the tail alone among the batch."""
+    from bpt_amd import kivi
+
+    print(f"kivi tail {tail_len} {tail_dtype} {layout} hq {q_heads}", flush=True)
+    lengths = [96, 0, 65]
+    dev, ref = make_cache(len(lengths), 8, 96, 8, seed=13)
+    q, qn = make_q(len(lengths), q_heads, 7)
+    tk, tv, tkn, tvn = tail_rows(len(lengths), 8, tail_len, 128, tail_dtype, 12)
+    if layout != "whole rows":
+        pad = 129 if layout == "odd token stride" else 136
+        store = torch.zeros((2, len(lengths), 8, tail_len, pad), dtype=tail_dtype, device="cuda")
+        at = 1 if layout == "odd offset" else 0
+        store[0, ..., at:at + 128], store[1, ..., at:at + 128] = tk, tv
+        tk, tv = store[0, ..., at:at + 128], store[1, ..., at:at + 128]
+    got = kivi.attend(q, dev, torch.tensor(lengths, dtype=torch.int32, device="cuda"), 0.1, tail=(tk, tv))
+    torch.cuda.synchronize()
+    close(got, want_step(qn, ref, lengths, tkn, tvn, 0.1), f"tail {tail_len} {tail_dtype} {layout}")
+
+
 @pytest.mark.parametrize("bits", [4, 16])
 def test_tail_on_the_float32_kernel(bits):
     """Head dim 64 (and a float32 bits-16 cache) take the float32 kernel; the tail is one more block there."""
