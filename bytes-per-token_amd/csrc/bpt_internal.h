@@ -143,12 +143,29 @@ constexpr int kMfmaMinRows = BPT_DECODE_MFMA_MIN_ROWS;
 constexpr int kMfmaMinRowsInt8 = BPT_DECODE_MFMA_MIN_ROWS_INT8;
 constexpr int kMfmaRows = 16;
 constexpr int kMfmaChunk = 32;
-// Many-row attention (decode_rows.h): chunks of kRowsChunk tokens, tiles of 32, 64 or 128 rows.
+// Many-row attention (decode_rows.h): chunks of kRowsChunk tokens, tiles of 32, 64, 128 or 256 rows. A 256-row tile
+// decodes each chunk once for twice the rows of a 128-row one and its waves share nothing, but its pieces are twice as
+// large: it is taken from kRowsWideChunks (tile, chunk) units on, eight per CU. Measured, 256 against 128 rows (us):
+// FP8 2048 + 2048 tokens, 16 heads (4096 units) 121 : 138; INT8 512 + 8192, 32 heads (4352) 165 : 191; FP8 150 + 12000,
+// 64 heads (3800) 132 : 152; FP8 3 x (40 + 2000), 32 heads (384) 35 : 35; FP8 100 + 1000, 16 heads (72) 26 : 23; BF16
+// 4 x 300, 32 heads (480) 51 : 47.
 constexpr int kRowsChunk = 128;
+constexpr int64_t kRowsWideChunks = 8 * kComputeUnits;
 constexpr int rows_tile(int rows) { return rows <= 32 ? 32 : rows <= 64 ? 64 : 128; }
 constexpr int rows_groups_per_cu(int tile) { return tile == 32 ? 2 : 1; }
 constexpr int kRowsMinChunks = 1;
 constexpr int kRowsPieceCost = 2;
+// Whether the pieces of split tiles are combined by a second launch: when a tile's partials (about grid / tiles + 1
+// pieces, no more than its chunks, of `tile` rows of 512 bytes) reach kRowsTwoPassBytes. Measured, one launch against
+// two (us): 64 + 4096 tokens, 16 heads (33 pieces of 64 KiB) 47.9 : 28.0; 3 x (40 + 2000), 32 heads (7 of 64) 39.8 : 35.6;
+// 2048 + 2048, 16 heads (3 of 128) 125 : 122; BF16 2 x 1024, 16 heads (2 of 64) 53 : 60; 4 x (33 + 300), 8 heads (3 of
+// 32) 17.4 : 19.4.
+constexpr int64_t kRowsTwoPassBytes = (int64_t)256 << 10;
+constexpr bool rows_two_pass(int64_t grid, int64_t tiles, int64_t chunks, int tile) {
+  if (grid <= 1 || tiles <= 0) return false;
+  const int64_t pieces = (grid + tiles - 1) / tiles + 1;
+  return (pieces < chunks ? pieces : chunks) * tile * kHeadDim * 4 >= kRowsTwoPassBytes;
+}
 // Largest tile line the kernel takes, in tiles and sequences of one KV head: 4-byte entries in LDS.
 constexpr int64_t kRowsMaxLine = 4096;
 // Waves per SIMD the matrix-core decode kernel is compiled for (its register budget: 512 / this).
@@ -180,6 +197,7 @@ struct DecodeParams {
   int piece_cost;      // line units charged per segment start (0 with a fixed split count)
   int equal_grid;      // > 0: if every sequence has the same length, the first equal_grid workgroups cut
                        // equal power-of-two partitions instead and the others leave
+  int two_pass;        // many-row kernel: split tiles are combined by a second launch (rows_two_pass)
   float qscale;      // sm_scale * log2(e)
   int q_dtype, out_dtype, table_i64;
   int noncausal;        // every query sees all of its sequence's tokens
@@ -341,6 +359,7 @@ hipError_t launch_decode_mfma(const DecodeParams& p, int kv_dtype, int scale_kin
 hipError_t launch_rows_32(const DecodeParams& p, int kv_dtype, int scale_kind, hipStream_t stream, const LaunchEvents& ev);
 hipError_t launch_rows_64(const DecodeParams& p, int kv_dtype, int scale_kind, hipStream_t stream, const LaunchEvents& ev);
 hipError_t launch_rows_128(const DecodeParams& p, int kv_dtype, int scale_kind, hipStream_t stream, const LaunchEvents& ev);
+hipError_t launch_rows_256(const DecodeParams& p, int kv_dtype, int scale_kind, hipStream_t stream, const LaunchEvents& ev);
 hipError_t launch_kivi(const KiviParams& p, int fmt, hipStream_t stream);
 // Any even head dim up to 256 and float32 bits-16 caches: one workgroup per (sequence, KV head, split).
 hipError_t launch_kivi_any(const KiviParams& p, int fmt, hipStream_t stream);

@@ -51,6 +51,7 @@ struct Plan {
   int equal_grid;  // workgroups that take equal partitions when all lengths are equal (0: none)
   int piece_cost;  // line units charged per segment start
   int waves;       // matrix-core kernel: waves per workgroup
+  bool two_pass;   // many-row kernel: a second launch combines the split tiles
   size_t ws_out_floats, ws_lse_floats, workspace, counters;
 };
 
@@ -70,8 +71,9 @@ bool takes_tiles(const bpt_decode_args* a, int rows, int tile) {
   return (int64_t)a->batch * (tiles + 1) <= bpt::kRowsMaxLine;
 }
 
-// tiles_ok: whether the many-row kernel may be chosen.
-int make_plan(const bpt_decode_args* a, Plan* pl, bool tiles_ok = true) {
+// tiles_ok: whether the many-row kernel may be chosen; wide_ok: and its 256-row tiles (whose partials outgrow the
+// device scratch of bpt_paged_decode_noalloc).
+int make_plan(const bpt_decode_args* a, Plan* pl, bool tiles_ok = true, bool wide_ok = true) {
   const char* fn = "bpt_decode_plan";
   if (!a) return fail(BPT_ERR_INVALID_ARGUMENT, "%s: args is NULL", fn);
   if (a->struct_size != sizeof(bpt_decode_args))
@@ -110,7 +112,12 @@ int make_plan(const bpt_decode_args* a, Plan* pl, bool tiles_ok = true) {
   // from 5 rows on (with fewer, the vector kernel reads each page once too and its INT8 decode is cheaper).
   pl->mfma = pl->rows <= bpt::kMfmaRows && ((a->kv_dtype == BPT_KV_FP8_E4M3FN && pl->rows >= bpt::kMfmaMinRows) ||
                                             (a->kv_dtype == BPT_KV_INT8 && pl->rows >= bpt::kMfmaMinRowsInt8));
-  const int tile = bpt::rows_tile(pl->rows);
+  int tile = bpt::rows_tile(pl->rows);
+  if (wide_ok && pl->rows > tile) {
+    const int64_t reach = (int64_t)a->max_blocks_per_seq * a->page_size;
+    const int64_t chunks = ((a->max_context < reach ? a->max_context : reach) + bpt::kRowsChunk - 1) / bpt::kRowsChunk;
+    if ((int64_t)((pl->rows + 255) / 256) * a->num_kv_heads * a->batch * chunks >= bpt::kRowsWideChunks) tile = 256;
+  }
   pl->tiles = tiles_ok && takes_tiles(a, pl->rows, tile);
   pl->rows_per_group = pl->tiles ? tile : pl->mfma ? bpt::kMfmaRows : (pl->rows <= 1 ? 1 : (pl->rows <= 2 ? 2 : 4));
   pl->n_rg = (pl->rows + pl->rows_per_group - 1) / pl->rows_per_group;
@@ -199,6 +206,7 @@ int make_plan(const bpt_decode_args* a, Plan* pl, bool tiles_ok = true) {
                    : a->batch == 1 ? 0
                    : pair ? bpt::kMfmaPairPieceCost
                    : (pl->mfma && pl->rows >= bpt::kManyRows ? bpt::kManyRowPieceCost : bpt::kDecodePieceCost);
+  pl->two_pass = pl->tiles && bpt::rows_two_pass(pl->grid, (int64_t)a->batch * pl->HR, max_nb, tile);
   // The many-row kernel's workgroups hold at most two partials each: the first and the last piece of their range.
   const size_t slots = pl->tiles ? 2 * (size_t)pl->grid : (size_t)a->batch * pl->HR + pl->grid;
   pl->ws_out_floats = slots * pl->rows_per_group * a->head_dim;
@@ -342,6 +350,7 @@ void line_fields(const Plan& pl, bpt::DecodeParams* p) {
   p->per_forced = pl.per_forced;
   p->equal_grid = pl.equal_grid;
   p->piece_cost = pl.piece_cost;
+  p->two_pass = pl.two_pass;
 }
 
 // Checks a decode call's arguments and buffers on the host and fills its launch parameters (*p, *pl); nothing
@@ -349,7 +358,7 @@ void line_fields(const Plan& pl, bpt::DecodeParams* p) {
 int decode_setup(const bpt_decode_args* a, const char* fn, const Buffers* own, bpt::DecodeParams* out, Plan* plan,
                  bool* empty) {
   Plan& pl = *plan;
-  int rc = make_plan(a, &pl);
+  int rc = make_plan(a, &pl, true, own == nullptr);
   if (rc) return rc;
   const Buffers buf = own ? *own : Buffers{a->workspace, a->workspace_bytes, a->counters, a->counters_bytes};
   *empty = a->batch == 0;
@@ -455,9 +464,10 @@ int paged_decode(const bpt_decode_args* a, void* stream, const bpt::LaunchEvents
     p.w_sq = fuse->s_sq;
     p.w_i64 = fuse->slot_i64;
   }
-  hipError_t e = pl.tiles  ? (pl.rows_per_group == 32   ? bpt::launch_rows_32
-                              : pl.rows_per_group == 64 ? bpt::launch_rows_64
-                                                        : bpt::launch_rows_128)(p, a->kv_dtype, a->scale_kind, (hipStream_t)stream, ev)
+  hipError_t e = pl.tiles  ? (pl.rows_per_group == 32    ? bpt::launch_rows_32
+                              : pl.rows_per_group == 64  ? bpt::launch_rows_64
+                              : pl.rows_per_group == 128 ? bpt::launch_rows_128
+                                                         : bpt::launch_rows_256)(p, a->kv_dtype, a->scale_kind, (hipStream_t)stream, ev)
                  : pl.mfma ? bpt::launch_decode_mfma(p, a->kv_dtype, a->scale_kind, (hipStream_t)stream, ev)
                            : bpt::launch_decode(p, a->kv_dtype, a->scale_kind, pl.rows_per_group, (hipStream_t)stream, ev);
   if (e != hipSuccess) return hip_fail(fn, e);
@@ -494,7 +504,7 @@ int bpt_set_tuning(const bpt_tuning* t) {
 // only form passed to kernels.
 namespace {
 
-constexpr size_t kScratchWorkspace = (size_t)34 << 20;  // the many-row kernel's largest: 512 slots of 128 rows
+constexpr size_t kScratchWorkspace = (size_t)34 << 20;  // the many-row kernel's largest here: 512 slots of 128 rows
 constexpr size_t kScratchCounters = (size_t)2 << 20;
 constexpr int kMaxDevices = 64;
 
@@ -538,7 +548,7 @@ extern "C" {
 int bpt_paged_decode_noalloc(const bpt_decode_args* a, void* stream) {
   const char* fn = "bpt_paged_decode_noalloc";
   Plan pl;
-  int rc = make_plan(a, &pl);
+  int rc = make_plan(a, &pl, true, false);
   if (rc) return rc;
   if (pl.workspace > kScratchWorkspace || pl.counters > kScratchCounters)
     return fail(BPT_ERR_INVALID_ARGUMENT,

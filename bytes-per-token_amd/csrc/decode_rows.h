@@ -17,11 +17,12 @@
 // fed to the MFMAs as f16 plus f16 remainder (FP8 / INT8 values, 22 bits) or as three bf16 parts (BF16 values, 24
 // bits); an f16 q over a BF16 cache as bf16 plus bf16 remainder (exact).
 //
-// What bounds it: at 128-row tiles the matrix cores (FP8: three products where two would do, for the weights' second
-// part) and, behind them, the softmax's VALU work; at 32 rows the first loads and the combine. Measured against the
-// vector kernel's 4-row groups, which decode every chunk rows / 4 times (8 KV heads, us): FP8 prompt chunks of 2048
-// over 2048 cached tokens, 16 heads 1898 -> 154; 32 over 0 22.9 -> 17.9; 16 over 16384 95 -> 58; verifies of 5 queries,
-// 32 heads, 16 sequences of 1024..3072 tokens 113 -> 37; BF16, 8 queries 208 -> 79; INT8, 5 queries, 64 heads 281 -> 48.
+// What bounds it: with many chunks the matrix cores (FP8: three products where two would do, for the weights' second
+// part) and the vector units behind them (256-row tiles, 2048 rows x 8 heads over 4096 tokens: 37 % and 52 % of the
+// cycles, and leaving out the second part, the exponentials or the decoding saves 15, 5 and 5 of 122 us); with few the
+// first loads and the partials. Measured against the vector kernel's 4-row groups, which decode every chunk rows / 4
+// times (8 KV heads, us): FP8 prompt chunks of 2048 over 2048 cached tokens, 16 heads 1885 -> 121; verifies of 5
+// queries, 32 heads, 16 sequences of 1024..3072 tokens 113 -> 34.
 //
 // LDS layouts (16-byte units; both spread the 8 lanes that one LDS cycle serves over all banks):
 //  * K: token row of 16 units, unit u at u ^ (token % 8) ^ (u / 8). Operand reads take one unit of 8 consecutive
@@ -53,7 +54,6 @@ struct RowsCfg {
   static constexpr int BM = 32 * WM;   // rows per tile
   static constexpr int CT = kRowsChunk;
   static constexpr int TW = CT / WN;               // tokens per wave and chunk
-  static constexpr int SUB = TW < 64 ? TW : 64;    // of which this many go through the softmax at once
   static constexpr bool kBf16 = KV == kKvBf16;
   static constexpr bool kF16K = QF16_ && !kBf16;   // K and q operands in f16 (an f16 q over codes), else bf16
   static constexpr bool kQSplit = QF16_ && kBf16;  // an f16 q as two bf16 parts
@@ -66,7 +66,7 @@ struct RowsCfg {
   static constexpr int kOut = BM * (kHeadDim + 4) * 4 + BM * 4;
   static constexpr int kSmem = NBUF * kBuf > kMerge ? (NBUF * kBuf > kOut ? NBUF * kBuf : kOut)
                                                     : (kMerge > kOut ? kMerge : kOut);
-  static_assert(NW % WM == 0 && TW % 32 == 0 && TW % SUB == 0 && (CT / 16) % NW == 0, "tile shape");
+  static_assert(NW % WM == 0 && TW % 32 == 0 && (CT / 16) % NW == 0, "tile shape");
 };
 
 // One chunk's codes of one thread, in flight.
@@ -304,103 +304,130 @@ struct RowsState {
   f32x16 o[4];
 };
 
-// Tokens [t0, t0 + SUB) of the chunk (T: their first token in the sequence) folded into the state. qs: the score
-// scale, not negative (SK token-head: in the per-token K scales instead). rlen: the tokens this lane's row sees;
-// masked: some row of the wave does not see all of them.
+// w0, w1 = f16 pairs hi + lo (22 bits): hi rounded to nearest, lo the rounded remainder. The remainders come from
+// v_fma_mix_f32, which reads a half as a float (the compiler converts back and subtracts: two instructions more each).
+__device__ __forceinline__ void rows_split_f16(float w0, float w1, uint32_t& hi, uint32_t& lo) {
+  const f16x2 h = {(_Float16)w0, (_Float16)w1};
+  hi = __builtin_bit_cast(uint32_t, h);
+  float r0, r1;
+  __asm__("v_fma_mix_f32 %0, %1, -1.0, %2 op_sel:[0,0,0] op_sel_hi:[1,0,0]" : "=v"(r0) : "v"(hi), "v"(w0));
+  __asm__("v_fma_mix_f32 %0, %1, -1.0, %2 op_sel:[1,0,0] op_sel_hi:[1,0,0]" : "=v"(r1) : "v"(hi), "v"(w1));
+  lo = __builtin_bit_cast(uint32_t, f16x2{(_Float16)r0, (_Float16)r1});
+}
+
+// The K operands (A) of 32 tokens from t0 on: one per 16 channels.
 template <typename C>
-__device__ __forceinline__ void rows_compute(const uint8_t* buf, const RowsScales<C>& ssc, int t0, int T, int lane,
-                                             const u32x4 (&qb)[C::kQOps], float qs, int rlen, bool masked, RowsState& st) {
-  constexpr int NS = C::SUB / 32;
+__device__ __forceinline__ void rows_read_k(const uint8_t* buf, int t0, int lane, u32x4 (&ka)[8]) {
   const int n = lane & 31, hf = lane >> 5;
   const uint8_t* kbuf = buf + (t0 + n) * 256;
-  const uint8_t* vbuf = buf + C::CT * kHeadDim * 2 + (t0 >> 6) * 16384 + n * 128;
-
-  f32x16 s[NS];
 #pragma unroll
-  for (int ns = 0; ns < NS; ++ns) {
+  for (int k = 0; k < 8; ++k) ka[k] = *(const u32x4*)(kbuf + 16 * ((2 * k + hf) ^ (n & 7) ^ (k >> 2)));
+}
+template <typename C>
+__device__ __forceinline__ f32x16 rows_scores(const u32x4 (&ka)[8], const u32x4 (&qb)[C::kQOps]) {
+  f32x16 s;
 #pragma unroll
-    for (int i = 0; i < 16; ++i) s[ns][i] = 0.0f;
-  }
+  for (int i = 0; i < 16; ++i) s[i] = 0.0f;
 #pragma unroll
   for (int k = 0; k < 8; ++k) {
-    const int un = 16 * ((2 * k + hf) ^ (n & 7) ^ (k >> 2));
-#pragma unroll
-    for (int ns = 0; ns < NS; ++ns) {
-      const u32x4 a = *(const u32x4*)(kbuf + ns * 32 * 256 + un);
-      s[ns] = rows_mfma_k<C>(a, qb[k], s[ns]);
-      if constexpr (C::kQSplit) s[ns] = rows_mfma_k<C>(a, qb[8 + k], s[ns]);
-    }
+    s = rows_mfma_k<C>(ka[k], qb[k], s);
+    if constexpr (C::kQSplit) s = rows_mfma_k<C>(ka[k], qb[8 + k], s);
   }
-
-  float vsc[NS][16];
-  float mul = qs;
-  float mx = kNegInf;
-  if constexpr (C::SK == kScaleTokenHead) {
-    mul = 1.0f;
+  return s;
+}
+// The V operands (A) of the 16 tokens from t0 on: one per 32 channels.
+template <typename C>
+__device__ __forceinline__ void rows_read_v(const uint8_t* buf, int t0, int lane, u32x4 (&va)[4]) {
+  const int n = lane & 31, hf = lane >> 5;
+  const uint8_t* vbuf = buf + C::CT * kHeadDim * 2 + (t0 >> 6) * 16384 + n * 128;
 #pragma unroll
-    for (int ns = 0; ns < NS; ++ns) {
+  for (int ct = 0; ct < 4; ++ct)
+    va[ct] = *(const u32x4*)(vbuf + ct * 4096 + 16 * ((2 * ((t0 & 63) >> 4) + hf) ^ ((n + (n >> 3)) & 7) ^ (4 * (ct & 1))));
+}
+
+// The wave's tokens [t0, t0 + TW) of the chunk (T: their first token in the sequence) folded into the state, 32 at a
+// time. qs: the score scale, not negative (SK token-head: in the per-token K scales instead). rlen: the tokens this
+// lane's row sees; rlen_min: the fewest that a row of the wave sees.
+//
+// Two waves share a SIMD, so LDS latency is covered by the wave itself: a block's V operands and the next block's K
+// operands are requested ahead of its softmax, and the next block's score products stand between its two halves.
+template <typename C>
+__device__ __forceinline__ void rows_compute(const uint8_t* buf, const RowsScales<C>& ssc, int t0, int T, int lane,
+                                             const u32x4 (&qb)[C::kQOps], float qs, int rlen, int rlen_min, RowsState& st) {
+  constexpr int NH = C::TW / 32;
+  const int hf = lane >> 5;
+  u32x4 ka[8];
+  rows_read_k<C>(buf, t0, lane, ka);
+  f32x16 s = rows_scores<C>(ka, qb);
+#pragma unroll
+  for (int half = 0; half < NH; ++half) {
+    const int th = t0 + 32 * half;
+    u32x4 va[2][4];
+    rows_read_v<C>(buf, th, lane, va[0]);
+
+    float mul = qs;
+    float mx = kNegInf;
+    if constexpr (C::SK == kScaleTokenHead) {
+      mul = 1.0f;
 #pragma unroll
       for (int a = 0; a < 4; ++a) {
-        const int at = t0 + 32 * ns + 8 * a + 4 * hf;
+        const int at = th + 8 * a + 4 * hf;
         const f32x4 kq = *(const f32x4*)&ssc[0][at];
-        const f32x4 vs = *(const f32x4*)&ssc[1][at];
 #pragma unroll
-        for (int j = 0; j < 4; ++j) {
-          s[ns][4 * a + j] *= kq[j];
-          vsc[ns][4 * a + j] = vs[j];
-        }
+        for (int j = 0; j < 4; ++j) s[4 * a + j] *= kq[j];
       }
     }
-  }
-  if (masked) {
-#pragma unroll
-    for (int ns = 0; ns < NS; ++ns) {
+    if (T + 32 * half + 32 > rlen_min) {  // some row of the wave does not see all of them
 #pragma unroll
       for (int i = 0; i < 16; ++i) {
-        const int tok = T + 32 * ns + 8 * (i >> 2) + 4 * hf + (i & 3);
-        const float x = C::SK == kScaleTokenHead ? s[ns][i] : s[ns][i] * qs;
-        s[ns][i] = tok < rlen ? x : kNegInf;
+        const int tok = T + 32 * half + 8 * (i >> 2) + 4 * hf + (i & 3);
+        const float x = C::SK == kScaleTokenHead ? s[i] : s[i] * qs;
+        s[i] = tok < rlen ? x : kNegInf;
       }
+      mul = 1.0f;
     }
-    mul = 1.0f;
-  }
-#pragma unroll
-  for (int ns = 0; ns < NS; ++ns) {
     if constexpr (C::SK == kScaleTokenHead) {
 #pragma unroll
       for (int a = 0; a < 4; ++a) {
-        const f32x4 vb = *(const f32x4*)&ssc[2][t0 + 32 * ns + 8 * a + 4 * hf];
+        const f32x4 vb = *(const f32x4*)&ssc[2][th + 8 * a + 4 * hf];
 #pragma unroll
-        for (int j = 0; j < 4; ++j) mx = fmaxf(mx, s[ns][4 * a + j] + vb[j]);
+        for (int j = 0; j < 4; ++j) mx = fmaxf(mx, s[4 * a + j] + vb[j]);
       }
     } else {
 #pragma unroll
-      for (int i = 0; i < 16; ++i) mx = fmaxf(mx, s[ns][i]);
+      for (int i = 0; i < 16; ++i) mx = fmaxf(mx, s[i]);
     }
-  }
-  mx = max_xor<32>(mx) * mul;
-  const bool move = mx > st.m + kSlack;
-  if (__any(move)) {
-    const float mn = move ? mx : st.m;
-    const float alpha = move ? fast_exp2(st.m - mn) : 1.0f;  // 0 when m was -inf
-    st.l *= alpha;
+    mx = max_xor<32>(mx) * mul;
+    const bool move = mx > st.m + kSlack;
+    if (__any(move)) {
+      const float mn = move ? mx : st.m;
+      const float alpha = move ? fast_exp2(st.m - mn) : 1.0f;  // 0 when m was -inf
+      st.l *= alpha;
 #pragma unroll
-    for (int ct = 0; ct < 4; ++ct) st.o[ct] *= alpha;
-    st.m = mn;
-  }
-  const float base = (st.m == kNegInf ? 0.0f : st.m) - kBias;
+      for (int ct = 0; ct < 4; ++ct) st.o[ct] *= alpha;
+      st.m = mn;
+    }
+    const float base = (st.m == kNegInf ? 0.0f : st.m) - kBias;
 
-  float l0 = 0.0f, l1 = 0.0f;
-#pragma unroll
-  for (int ns = 0; ns < NS; ++ns) {
+    if (half + 1 < NH) rows_read_k<C>(buf, th + 32, lane, ka);
+    rows_read_v<C>(buf, th + 16, lane, va[1]);
+    f32x16 s_next = s;
+    float l0 = 0.0f, l1 = 0.0f;
 #pragma unroll
     for (int h2 = 0; h2 < 2; ++h2) {
       float w[8];
 #pragma unroll
       for (int j = 0; j < 8; ++j) {
-        const float e = fast_exp2(fmaf(s[ns][8 * h2 + j], mul, -base));
-        if (j & 1) l1 += e; else l0 += e;
-        w[j] = C::SK == kScaleTokenHead ? e * vsc[ns][8 * h2 + j] : e;
+        w[j] = fast_exp2(fmaf(s[8 * h2 + j], mul, -base));
+        if (j & 1) l1 += w[j]; else l0 += w[j];
+      }
+      if constexpr (C::SK == kScaleTokenHead) {
+#pragma unroll
+        for (int a = 0; a < 2; ++a) {
+          const f32x4 vs = *(const f32x4*)&ssc[1][th + 16 * h2 + 8 * a + 4 * hf];
+#pragma unroll
+          for (int j = 0; j < 4; ++j) w[4 * a + j] *= vs[j];
+        }
       }
       u32x4 part[3];
       if constexpr (C::kBf16) {
@@ -417,27 +444,22 @@ __device__ __forceinline__ void rows_compute(const uint8_t* buf, const RowsScale
       } else {
 #pragma unroll
         for (int j = 0; j < 4; ++j) {
-          const f16x2 x = {(_Float16)w[2 * j], (_Float16)w[2 * j + 1]};
-          const f16x2 r = {(_Float16)(w[2 * j] - (float)x.x), (_Float16)(w[2 * j + 1] - (float)x.y)};
-          part[0][j] = __builtin_bit_cast(uint32_t, x);
-          part[1][j] = __builtin_bit_cast(uint32_t, r);
+          uint32_t hi, lo;
+          rows_split_f16(w[2 * j], w[2 * j + 1], hi, lo);
+          part[0][j] = hi;
+          part[1][j] = lo;
         }
-      }
-      const int s16 = 2 * ns + h2;  // t0 is a multiple of SUB: inside its 64-token block
-      u32x4 a[4];
-#pragma unroll
-      for (int ct = 0; ct < 4; ++ct) {
-        const int un = (2 * (((t0 & 63) >> 4) + s16) + hf) ^ ((n + (n >> 3)) & 7) ^ (4 * (ct & 1));
-        a[ct] = *(const u32x4*)(vbuf + ct * 4096 + 16 * un);
       }
 #pragma unroll
       for (int q = 0; q < (C::kBf16 ? 3 : 2); ++q) {
 #pragma unroll
-        for (int ct = 0; ct < 4; ++ct) st.o[ct] = rows_mfma_v<C>(a[ct], part[q], st.o[ct]);
+        for (int ct = 0; ct < 4; ++ct) st.o[ct] = rows_mfma_v<C>(va[h2][ct], part[q], st.o[ct]);
       }
+      if (h2 == 0 && half + 1 < NH) s_next = rows_scores<C>(ka, qb);
     }
+    st.l += l0 + l1;
+    s = s_next;
   }
-  st.l += l0 + l1;
 }
 
 // Row gr's q as the B operands of the score products (channels 16 k + 8 hf .. + 7); flip: negated.
@@ -589,6 +611,74 @@ __device__ __forceinline__ void rows_combine(const DecodeParams& p, int b, int h
   }
 }
 
+// The combine as a launch of its own (DecodeParams::two_pass): the workgroups take strips of kCombineRows rows of the
+// tiles in turn, the pieces in the slots of rows_combine. The last arriver of a tile is one CU, which reads some 50 GB/s
+// past the L2s, so 33 pieces of 128 rows (2 MiB) took it about 25 us. Spread over the chip they take 5.5 us: a call whose
+// tiles have much to combine pays a second launch instead (rows_two_pass), and its pieces are plain stores.
+constexpr int kCombineRows = 8, kCombineWaves = 4, kCombineGrid = 4 * kComputeUnits;
+template <int BM>
+__global__ __launch_bounds__(kCombineWaves * 64) void rows_combine_kernel(const DecodeParams p) {
+  constexpr int D = kHeadDim, NT = kCombineWaves * 64, kJ = 8;
+  static_assert(NT == kCombineRows * (D / 4), "one output of four channels per thread");
+  extern __shared__ int s_dyn[];
+  __shared__ int s_wsum[kCombineWaves];
+  const int T = p.n_rg, X = p.piece_cost, tid = threadIdx.x;
+  int* s_line = s_dyn;
+  int* s_len = s_dyn + p.B * T + 1;
+  build_tile_line<kCombineWaves, BM>(p, s_line, s_len, s_wsum);
+  const int64_t total = (int64_t)p.Hkv * s_line[p.B * T];
+  const int64_t per = p.per_forced > 0 ? p.per_forced : (total + p.grid - 1) / p.grid;
+  const bool packed = !p.merge_out && !p.lse_out && p.out_dtype != kFF32 && ((uintptr_t)p.out & 7) == 0 &&
+                      ((p.o_sb | p.o_sq | p.o_sh) & 3) == 0;
+  constexpr int kStrips = BM / kCombineRows;
+  const int ch = 4 * (tid % (D / 4));
+  for (int64_t strip = blockIdx.x; strip < (int64_t)p.B * p.Hkv * T * kStrips; strip += gridDim.x) {
+    const int tile = (int)(strip / kStrips);
+    const int r = (int)(strip % kStrips) * kCombineRows + tid / (D / 4);
+    const int t = tile % T, h = tile / T % p.Hkv, b = tile / (T * p.Hkv);
+    const int gr = t * BM + r;
+    if (s_len[b] == 0 || gr >= p.Q * p.G) continue;
+    const int start = s_line[b * T + t], end = s_line[b * T + t + 1];
+    const int64_t c0 = (int64_t)p.Hkv * s_line[b * T] + (int64_t)h * (s_line[(b + 1) * T] - s_line[b * T]) + (start - s_line[b * T]);
+    const int64_t g_first = (c0 + X) / per;
+    const int n = (int)((c0 + (end - start) - 1) / per - g_first) + 1;
+    if (n == 1) continue;  // written by the workgroup that held it
+    float M = kNegInf, W = 0.0f;
+    f32x4 O = {0.0f, 0.0f, 0.0f, 0.0f};
+    for (int j0 = 0; j0 < n; j0 += kJ) {
+      float lv[kJ];
+      f32x4 ov[kJ];
+#pragma unroll
+      for (int j = 0; j < kJ; ++j) {
+        const int jj = min(j0 + j, n - 1);  // a piece past the last is read again and weighs nothing
+        const int64_t row = (2 * (g_first + jj) + (jj == 0 ? 1 : 0)) * BM + r;
+        lv[j] = p.ws_lse[row];
+        ov[j] = *(const f32x4*)(p.ws_out + row * D + ch);
+      }
+      float nm = M;
+#pragma unroll
+      for (int j = 0; j < kJ; ++j) {
+        if (j0 + j >= n) lv[j] = kNegInf;
+        nm = fmaxf(nm, lv[j]);
+      }
+      const float mu = nm == kNegInf ? 0.0f : nm;
+      const float alpha = W > 0.0f ? fast_exp2(M - mu) : 0.0f;
+      W *= alpha;
+      O *= alpha;
+#pragma unroll
+      for (int j = 0; j < kJ; ++j) {
+        const float e = fast_exp2(lv[j] - mu);  // 0 for pieces in which the row saw no token
+        W += e;
+        O += ov[j] * e;
+      }
+      M = nm;
+    }
+    const int qi = gr / p.G;
+    const float inv = W > 0.0f ? 1.0f / W : 0.0f;
+    rows_write4(p, b, qi, h * p.G + (gr - qi * p.G), ch, O * inv, W > 0.0f ? M + __log2f(W) : kNegInf, packed);
+  }
+}
+
 template <int KV, int SK, bool PU, bool QF16, int WM, int NW, int NBUF>
 __global__ __launch_bounds__(NW * 64, 2) void decode_rows_kernel(const DecodeParams p) {
   typedef RowsCfg<KV, SK, PU, QF16, WM, NW, NBUF> C;
@@ -713,31 +803,33 @@ __global__ __launch_bounds__(NW * 64, 2) void decode_rows_kernel(const DecodePar
       __syncthreads();
     }
     for (int kk = k; kk < k_end; ++kk) {
+      // The lane's LDS and cache offsets are worked out again for every chunk (some 50 instructions): kept over the
+      // loop they would take 40 registers that the operands in flight need.
+      int ln = lane;
+      __asm__ volatile("" : "+v"(ln));
       if constexpr (NBUF == 1) {
         if (kk > k) __syncthreads();  // every wave is done with the previous chunk
-        rows_store<C>(p, stage, smem, s_sc[0], wave, lane, tid);
+        rows_store<C>(p, stage, smem, s_sc[0], wave, ln, tid);
         __syncthreads();
       }
       const bool last = kk + 1 == k_end;
       if (!last) {
-        rows_issue<C>(p, b, h, kk + 1, len, wave, lane, tid, stage);
+        rows_issue<C>(p, b, h, kk + 1, len, wave, ln, tid, stage);
         rows_fetch_pages<C>(p, b, kk + 2, len, wave, tid, stage);
       } else if (more) {
         rows_fetch_pages<C>(p, nb_, 0, nlen, wave, tid, stage);
-        rows_issue<C>(p, nb_, nh, 0, nlen, wave, lane, tid, stage);
+        rows_issue<C>(p, nb_, nh, 0, nlen, wave, ln, tid, stage);
         rows_fetch_pages<C>(p, nb_, 1, nlen, wave, tid, stage);
       }
-#pragma unroll
-      for (int sub = 0; sub < C::TW / C::SUB; ++sub) {
-        const int t0 = wn * C::TW + sub * C::SUB;
+      {
+        const int t0 = wn * C::TW;
         const int tok = kk * C::CT + t0;
-        if (tok < rlen_max)
-          rows_compute<C>(smem + cur * C::kBuf, s_sc[cur], t0, tok, lane, qb, fabsf(qscale), rlen, tok + C::SUB > rlen_min, st);
+        if (tok < rlen_max) rows_compute<C>(smem + cur * C::kBuf, s_sc[cur], t0, tok, ln, qb, fabsf(qscale), rlen, rlen_min, st);
       }
       if constexpr (NBUF == 2) {
         if (!last) {
           cur ^= 1;
-          rows_store<C>(p, stage, smem + cur * C::kBuf, s_sc[cur], wave, lane, tid);
+          rows_store<C>(p, stage, smem + cur * C::kBuf, s_sc[cur], wave, ln, tid);
           __syncthreads();
         }
       }
@@ -820,13 +912,16 @@ __global__ __launch_bounds__(NW * 64, 2) void decode_rows_kernel(const DecodePar
         const int row = t * BM + r;
         const int qi = row / p.G;
         rows_write4(p, b, qi, h * p.G + (row - qi * p.G), ch, o, s_lse[r], packed);
+      } else if (p.two_pass) {
+        *(f32x4*)(p.ws_out + (slot * BM + r) * D + ch) = o;
+        if (ch == 0) p.ws_lse[slot * BM + r] = s_lse[r];
       } else {
         ws_store2(p.ws_out + (slot * BM + r) * D + ch, o[0], o[1]);
         ws_store2(p.ws_out + (slot * BM + r) * D + ch + 2, o[2], o[3]);
         if (ch == 0) ws_store(p.ws_lse + slot * BM + r, s_lse[r]);
       }
     }
-    if (!whole) {
+    if (!whole && !p.two_pass) {
       const int seg = (b * Hkv + h) * T + t;
       const int n = (int)(g_last - g_first + 1);
       ws_publish();
@@ -852,14 +947,23 @@ __global__ __launch_bounds__(NW * 64, 2) void decode_rows_kernel(const DecodePar
 }
 
 template <int KV, int SK, int WM, int NW, int NBUF>
-static hipError_t launch_rows_t(const DecodeParams& p, hipStream_t stream, const LaunchEvents& ev) {
+static hipError_t launch_rows_t(const DecodeParams& p, hipStream_t stream, const LaunchEvents& events) {
   dim3 grid(p.grid), block(NW * 64);
   const size_t lds = (size_t)(p.B * p.n_rg + 1 + p.B) * sizeof(int);
   const bool pu = p.P >= 16, f16 = p.q_dtype == kFF16;
+  LaunchEvents ev = events;  // the interval of a call spans both of its launches
+  if (p.two_pass) ev.stop = nullptr;
   if (pu && !f16) launch_kernel(decode_rows_kernel<KV, SK, true, false, WM, NW, NBUF>, grid, block, lds, stream, ev, p);
   else if (pu) launch_kernel(decode_rows_kernel<KV, SK, true, true, WM, NW, NBUF>, grid, block, lds, stream, ev, p);
   else if (!f16) launch_kernel(decode_rows_kernel<KV, SK, false, false, WM, NW, NBUF>, grid, block, lds, stream, ev, p);
   else launch_kernel(decode_rows_kernel<KV, SK, false, true, WM, NW, NBUF>, grid, block, lds, stream, ev, p);
+  hipError_t e = hipGetLastError();
+  if (e != hipSuccess || !p.two_pass) return e;
+  constexpr int BM = 32 * WM;
+  const int64_t strips = (int64_t)p.B * p.Hkv * p.n_rg * (BM / kCombineRows);
+  dim3 cgrid((unsigned)(strips < kCombineGrid ? strips : kCombineGrid)), cblock(kCombineWaves * 64);
+  if (events.start) hipExtLaunchKernelGGL((rows_combine_kernel<BM>), cgrid, cblock, (uint32_t)lds, stream, nullptr, events.stop, 0u, p);
+  else hipLaunchKernelGGL((rows_combine_kernel<BM>), cgrid, cblock, lds, stream, p);
   return hipGetLastError();
 }
 

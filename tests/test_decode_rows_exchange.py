@@ -17,13 +17,14 @@ def test_partial_exchange_sequence(tmp_path):
 
 
 @pytest.mark.parametrize("fmt", ["fp8", "int8", "bf16"])
-@pytest.mark.parametrize("nq,hq,tile", [(9, 16, 32), (16, 16, 32), (17, 16, 64), (8, 64, 64), (65, 8, 128), (2048, 64, 128)])
+@pytest.mark.parametrize("nq,hq,tile", [(9, 16, 32), (16, 16, 32), (17, 16, 64), (8, 64, 64), (65, 8, 128), (255, 8, 128), (256, 64, 256), (2048, 64, 256)])
 def test_plan_takes_tiles_from_17_rows(built_lib, fmt, nq, hq, tile):
     q, k, v, table, lens, ks, vs = cpu_case(fmt, b=2, nq=nq, hq=hq, max_blocks=256, nb=8192)
     grid, chunk, ws, cnt = decode_plan(q, k, v, table, lens, ks, vs, scale=0.1, max_context=4096)
     tiles = -(-nq * (hq // 8) // tile)
     assert chunk == 128 and cnt == align256(2 * 8 * tiles * 4)
-    assert ws == align256(2 * grid * tile * 129 * 4) and ws <= 34 << 20  # the no-allocation array holds any such call
+    assert ws == align256(2 * grid * tile * 129 * 4)  # the no-allocation array (34 MiB) holds any call with 128-row tiles
+    assert tile == 256 or ws <= 34 << 20
     assert grid == min(256 * (2 if tile == 32 else 1), 2 * 8 * tiles * 32)
 
 

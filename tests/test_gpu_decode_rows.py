@@ -1,6 +1,6 @@
 """GPU: the many-row kernel (more than 16 query rows per KV head, decode_rows.h) against the oracle.
 
-Sizes sit at the edges of its tiles (32, 64 and 128 rows), chunks (128 tokens) and pages. bf16 results at the decode
+Sizes sit at the edges of its tiles (32, 64, 128 and 256 rows), chunks (128 tokens) and pages. bf16 results at the decode
 tolerance; float32 results within 2^-14 of the largest output: the value weights carry at least 22 bits, so what is
 left is the float32 rounding of scores up to 2^7 base-2 units (2^-18 each, on both sides: a weight off by up to
 2^-17 ln 2 in the kernel and in the oracle, times the few that accumulate).
@@ -33,6 +33,45 @@ def test_rows_page_sizes_and_q_dtypes(fmt, scales, page, q_dtype):
     c = make_case(fmt, [300, 77], hq=8, hkv=2, nq=9, page=page, scales=scales, seed=page, table_dtype=torch.int64)
     got, want = run_case(c, q=c["q"].to(q_dtype), out_dtype=q_dtype)
     check(got, want, f"{fmt}/{scales} page {page} {q_dtype}")
+
+
+@pytest.mark.parametrize("fmt,scales", FORMATS)
+@pytest.mark.parametrize("nq,q_dtype", [(256, torch.bfloat16), (257, torch.float16), (300, torch.bfloat16)])
+def test_rows_wide_tiles(fmt, scales, nq, q_dtype):
+    """256-row tiles, pieces combined by the second launch: 1024 rows per KV head are four whole tiles, 1028 and 1200
+    leave a part of one; sequences of no tokens, of the new ones alone and of some more."""
+    from bpt_amd import decode_plan
+
+    c = make_case(fmt, [2900, 0, nq, 700], hq=32, hkv=8, nq=nq, scales=scales, seed=nq)
+    plan = decode_plan(c["q"], c["k"], c["v"], c["table"], c["lens"], c["ks"], c["vs"], scale=0.1, max_context=2900)
+    assert plan[2] >= 2 * plan[0] * 256 * 129 * 4  # 256-row slots
+    got, want = run_case(c, q=c["q"].to(q_dtype), out_dtype=q_dtype)
+    check(got, want, f"{fmt}/{scales} {nq} queries {q_dtype}")
+
+
+@pytest.mark.parametrize("nq", [40, 100])
+def test_rows_two_launches_replay_in_a_graph(nq):
+    """Both launches under capture, replayed with eager work between: the partials of one replay are not the next's."""
+    from bpt_amd import paged_decode_attention
+
+    c = make_case("fp8", [3000, 450], hq=16, hkv=2, nq=nq, seed=nq)
+    args = (c["q"], c["k"], c["v"], c["table"], c["lens"], c["ks"], c["vs"])
+    want = paged_decode_attention(*args, scale=0.09, max_context=3000)
+    out = torch.empty_like(want)
+    stream = torch.cuda.Stream()
+    with torch.cuda.stream(stream):
+        paged_decode_attention(*args, scale=0.09, max_context=3000, out=out)
+    torch.cuda.synchronize()
+    graph = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(graph, stream=stream):
+        paged_decode_attention(*args, scale=0.09, max_context=3000, out=out)
+    for _ in range(3):
+        out.zero_()
+        graph.replay()
+        torch.cuda.synchronize()
+        assert torch.equal(out, want)
+        paged_decode_attention(*args, scale=0.09, max_context=3000)
+        torch.cuda.synchronize()
 
 
 @pytest.mark.parametrize("num_splits", [1, 3, 1000])
