@@ -98,6 +98,7 @@ class DecodeArgs(ctypes.Structure):
     ]
 
 
+DECODE_ARGS_SIZE = ctypes.sizeof(DecodeArgs)
 DECODE_NONCAUSAL = 1
 
 
@@ -136,6 +137,7 @@ class AppendArgs(ctypes.Structure):
     ]
 
 
+APPEND_ARGS_SIZE = ctypes.sizeof(AppendArgs)
 KIVI_INT4, KIVI_INT8, KIVI_F16, KIVI_BF16, KIVI_F32 = 0, 1, 2, 3, 4
 
 

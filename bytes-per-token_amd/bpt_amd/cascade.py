@@ -26,7 +26,7 @@ from __future__ import annotations
 import torch
 
 from ._lib import DECODE_NONCAUSAL
-from .paged_attention import _require, paged_decode_attention
+from .paged_attention import paged_decode_attention
 
 
 def _rows_per_pass(total_queries: int, heads_per_kv: int) -> int:
@@ -67,22 +67,28 @@ def cascade_decode_attention(
     q4 = q[:, None] if squeeze else q
     b, nq, hq, d = q4.shape
     hkv, page = k_cache.shape[2], k_cache.shape[1]
-    _require(hq % hkv == 0, f"{hq} query heads are not a multiple of {hkv} KV heads")
+    if not (hq % hkv == 0):
+        raise ValueError(f"{hq} query heads are not a multiple of {hkv} KV heads")
     heads_per_kv = hq // hkv
-    _require(prefix_pages >= 1, "prefix_pages must be at least 1 (use paged_decode_attention without a prefix)")
-    _require(block_table.dim() == 2 and block_table.shape[1] >= prefix_pages,
-             f"block_table must hold at least the {prefix_pages} prefix pages")
+    if not (prefix_pages >= 1):
+        raise ValueError("prefix_pages must be at least 1 (use paged_decode_attention without a prefix)")
+    if not (block_table.dim() == 2 and block_table.shape[1] >= prefix_pages):
+        raise ValueError(f"block_table must hold at least the {prefix_pages} prefix pages")
     prefix = prefix_pages * page
-    _require(max_context >= prefix, f"max_context {max_context} is shorter than the {prefix}-token prefix")
+    if not (max_context >= prefix):
+        raise ValueError(f"max_context {max_context} is shorter than the {prefix}-token prefix")
     groups = [(0, b)] if groups is None else [(int(s), int(e)) for s, e in groups]
     at = 0
     for s, e in groups:
-        _require(s == at and e > s, "groups must be consecutive, non-empty [start, end) ranges covering the batch")
+        if not (s == at and e > s):
+            raise ValueError("groups must be consecutive, non-empty [start, end) ranges covering the batch")
         at = e
-    _require(at == b, "groups must cover the whole batch")
+    if not (at == b):
+        raise ValueError("groups must cover the whole batch")
     if context_lens_host is not None:
         short = [i for i, n in enumerate(context_lens_host) if n < prefix + nq - 1]
-        _require(not short, f"sequences {short[:8]} end inside the shared prefix: their queries would see all of it")
+        if not (not short):
+            raise ValueError(f"sequences {short[:8]} end inside the shared prefix: their queries would see all of it")
     dev = q4.device
     q4c = q4 if q4.stride(0) == nq * q4.stride(1) and q4.stride(1) == hq * q4.stride(2) and q4.stride(2) == d else q4.contiguous()
 

@@ -36,7 +36,7 @@ import torch
 
 from . import _lib
 from ._lib import F_BF16, F_F16, F_F32, KIVI_BF16, KIVI_F16, KIVI_F32, KIVI_INT4, KIVI_INT8
-from .paged_attention import cached_buffer
+from .paged_attention import _stream, cached_buffer
 
 _Q_CODES = {torch.bfloat16: F_BF16, torch.float16: F_F16, torch.float32: F_F32}
 
@@ -103,18 +103,18 @@ def quantize_kv_into(k: torch.Tensor, v: torch.Tensor, kv: Any, start: int) -> N
     caches get the values copied. Integration/kv_cache.py:147-156 does this with reference.quantize_kv and
     slice assignments."""
     b, h, n, d = k.shape
-    _require(tuple(v.shape) == (b, h, n, d) and v.dtype == k.dtype and v.stride() == k.stride(),
-             "k and v must be [B, Hkv, n, D] with one dtype and layout")
-    _require(kv.k_codes.shape[0] == b and kv.k_codes.shape[1] == h, "the cache's batch and KV heads must match")
-    _require(start >= 0 and start % kv.group == 0 and start + n <= kv.k_codes.shape[2],
-             f"tokens {start} .. {start + n} must start on a key group and fit the cache")
+    if not (tuple(v.shape) == (b, h, n, d) and v.dtype == k.dtype and v.stride() == k.stride()):
+        raise ValueError("k and v must be [B, Hkv, n, D] with one dtype and layout")
+    if not (kv.k_codes.shape[0] == b and kv.k_codes.shape[1] == h):
+        raise ValueError("the cache's batch and KV heads must match")
+    if not (start >= 0 and start % kv.group == 0 and start + n <= kv.k_codes.shape[2]):
+        raise ValueError(f"tokens {start} .. {start + n} must start on a key group and fit the cache")
     if kv.bits == 16:
         kv.k_codes[:, :, start:start + n].copy_(k)
         kv.v_codes[:, :, start:start + n].copy_(v)
         return
     a = quantize_args(k, v, kv, start)
-    stream = torch.cuda.current_stream(k.device).cuda_stream
-    _lib.check(_lib.lib().bpt_kivi_quantize(ctypes.byref(a), ctypes.c_void_p(stream)))
+    _lib.check(_lib.lib().bpt_kivi_quantize(a, _stream(k.device)))
 
 
 def quantize_args(k: torch.Tensor, v: torch.Tensor, kv: Any, start: int) -> Any:
@@ -122,28 +122,39 @@ def quantize_args(k: torch.Tensor, v: torch.Tensor, kv: Any, start: int) -> Any:
     caller that launches the same write again without the Python checks (a timing loop, a captured graph).
     The struct holds raw pointers: the tensors must stay alive and in place while it is used."""
     b, h, n, d = k.shape
-    _require(tuple(v.shape) == (b, h, n, d) and v.dtype == k.dtype and v.stride() == k.stride(),
-             "k and v must be [B, Hkv, n, D] with one dtype and layout")
-    _require(kv.k_codes.shape[0] == b and kv.k_codes.shape[1] == h, "the cache's batch and KV heads must match")
-    _require(start >= 0 and start % kv.group == 0 and start + n <= kv.k_codes.shape[2],
-             f"tokens {start} .. {start + n} must start on a key group and fit the cache")
-    _require(kv.bits in (4, 8), f"bits must be 4, 8 or 16, got {kv.bits}")
-    _require(n % kv.group == 0, f"{n} tokens are not a whole number of groups of {kv.group}")
-    _require(k.dtype in _Q_CODES and k.stride(-1) == 1, "k and v must be bf16, f16 or f32 with contiguous channels")
+    if not (tuple(v.shape) == (b, h, n, d) and v.dtype == k.dtype and v.stride() == k.stride()):
+        raise ValueError("k and v must be [B, Hkv, n, D] with one dtype and layout")
+    if not (kv.k_codes.shape[0] == b and kv.k_codes.shape[1] == h):
+        raise ValueError("the cache's batch and KV heads must match")
+    if not (start >= 0 and start % kv.group == 0 and start + n <= kv.k_codes.shape[2]):
+        raise ValueError(f"tokens {start} .. {start + n} must start on a key group and fit the cache")
+    if not (kv.bits in (4, 8)):
+        raise ValueError(f"bits must be 4, 8 or 16, got {kv.bits}")
+    if not (n % kv.group == 0):
+        raise ValueError(f"{n} tokens are not a whole number of groups of {kv.group}")
+    if not (k.dtype in _Q_CODES and k.stride(-1) == 1):
+        raise ValueError("k and v must be bf16, f16 or f32 with contiguous channels")
     dev = k.device
-    _require(dev.type == "cuda", "quantize_kv runs on a GPU: k must be a cuda tensor")
+    if not (dev.type == "cuda"):
+        raise ValueError("quantize_kv runs on a GPU: k must be a cuda tensor")
     kc = kv.k_codes[:, :, start:start + n]
     vc = kv.v_codes[:, :, start:start + n]
     g0, g1 = start // kv.group, (start + n) // kv.group
     ks, kz = kv.k_scale[:, :, g0:g1], kv.k_zero[:, :, g0:g1]
     vs, vz = kv.v_scale[:, :, start:start + n], kv.v_zero[:, :, start:start + n]
-    _require(kc.dtype == torch.uint8 and kc.stride() == vc.stride() and kc.stride(-1) == 1, "codes: uint8, shared layout")
-    _require(kc.shape[3] * (2 if kv.bits == 4 else 1) == d, f"codes hold {kc.shape[3]} bytes per token, k has D={d}")
-    _require(all(t.dtype == torch.float16 for t in (ks, kz, vs, vz)), "grids must be float16")
-    _require(ks.stride() == kz.stride() and ks.stride(-1) == 1, "key grids: shared layout, contiguous channels")
-    _require(vs.stride() == vz.stride() and vs.stride(-1) == 1, "value grids: shared layout, unit token stride")
+    if not (kc.dtype == torch.uint8 and kc.stride() == vc.stride() and kc.stride(-1) == 1):
+        raise ValueError("codes: uint8, shared layout")
+    if not (kc.shape[3] * (2 if kv.bits == 4 else 1) == d):
+        raise ValueError(f"codes hold {kc.shape[3]} bytes per token, k has D={d}")
+    if not (all(t.dtype == torch.float16 for t in (ks, kz, vs, vz))):
+        raise ValueError("grids must be float16")
+    if not (ks.stride() == kz.stride() and ks.stride(-1) == 1):
+        raise ValueError("key grids: shared layout, contiguous channels")
+    if not (vs.stride() == vz.stride() and vs.stride(-1) == 1):
+        raise ValueError("value grids: shared layout, unit token stride")
     for t in (v, kc, vc, ks, kz, vs, vz):
-        _require(t.device == dev, f"every tensor must be on {dev}")
+        if not (t.device == dev):
+            raise ValueError(f"every tensor must be on {dev}")
     a = _lib.KiviQuantArgs()
     a.struct_size = ctypes.sizeof(_lib.KiviQuantArgs)
     a.bits, a.src_dtype = kv.bits, _Q_CODES[k.dtype]
@@ -164,11 +175,6 @@ def default_split(batch: int, kv_heads: int, tokens: int, group: int = 32, max_p
     `max_programs` (sequence, KV head, split) units; a power of two."""
     per_program = max(tokens * batch * kv_heads // max_programs, 4 * group)
     return max(group, 1 << (per_program.bit_length() - 1))
-
-
-def _require(cond: bool, msg: str) -> None:
-    if not cond:
-        raise ValueError(msg)
 
 
 def _format(kv: Any) -> int:
@@ -192,24 +198,33 @@ def _launch(q, kv, lengths, scale, split, n_splits, out, lse, tail=None) -> None
     fmt = _format(kv)
     b, hq, d = q.shape
     kc, vc = kv.k_codes, kv.v_codes
-    _require(kc.dim() == 4 and kc.shape == vc.shape, "k_codes and v_codes must be [B, Hkv, T, E] of one shape")
-    _require(kc.shape[0] == b, f"the cache holds {kc.shape[0]} sequences, q {b}")
+    if not (kc.dim() == 4 and kc.shape == vc.shape):
+        raise ValueError("k_codes and v_codes must be [B, Hkv, T, E] of one shape")
+    if not (kc.shape[0] == b):
+        raise ValueError(f"the cache holds {kc.shape[0]} sequences, q {b}")
     hkv, t_max = kc.shape[1], kc.shape[2]
     quant = fmt in (KIVI_INT4, KIVI_INT8)
     if quant:
-        _require(kc.dtype == torch.uint8 and vc.dtype == torch.uint8, "4- and 8-bit codes must be uint8")
-        _require(kc.shape[3] * (2 if fmt == KIVI_INT4 else 1) == d, f"codes hold {kc.shape[3]} bytes per token, q has D={d}")
+        if not (kc.dtype == torch.uint8 and vc.dtype == torch.uint8):
+            raise ValueError("4- and 8-bit codes must be uint8")
+        if not (kc.shape[3] * (2 if fmt == KIVI_INT4 else 1) == d):
+            raise ValueError(f"codes hold {kc.shape[3]} bytes per token, q has D={d}")
     else:
-        _require(vc.dtype == kc.dtype and kc.shape[3] == d, "bits-16 keys and values must share q's head dim and a dtype")
-    _require(q.dtype in _Q_CODES, f"q must be bfloat16, float16 or float32, got {q.dtype}")
-    _require(q.stride(-1) == 1 and kc.stride(-1) == 1 and vc.stride() == kc.stride(), "channels must be contiguous")
-    _require(lengths.dtype == torch.int32 and tuple(lengths.shape) == (b,) and lengths.is_contiguous(),
-             f"lengths must be int32 [{b}]")
+        if not (vc.dtype == kc.dtype and kc.shape[3] == d):
+            raise ValueError("bits-16 keys and values must share q's head dim and a dtype")
+    if not (q.dtype in _Q_CODES):
+        raise ValueError(f"q must be bfloat16, float16 or float32, got {q.dtype}")
+    if not (q.stride(-1) == 1 and kc.stride(-1) == 1 and vc.stride() == kc.stride()):
+        raise ValueError("channels must be contiguous")
+    if not (lengths.dtype == torch.int32 and tuple(lengths.shape) == (b,) and lengths.is_contiguous()):
+        raise ValueError(f"lengths must be int32 [{b}]")
     dev = q.device
-    _require(dev.type == "cuda", "decode_attention runs on a GPU: q must be a cuda tensor")
+    if not (dev.type == "cuda"):
+        raise ValueError("decode_attention runs on a GPU: q must be a cuda tensor")
     grids = (kv.k_scale, kv.k_zero, kv.v_scale, kv.v_zero) if quant else ()
     for t in (kc, vc, lengths, *grids):
-        _require(t.device == dev, f"every tensor must be on {dev}")
+        if not (t.device == dev):
+            raise ValueError(f"every tensor must be on {dev}")
 
     a = _lib.KiviArgs()
     a.struct_size = ctypes.sizeof(_lib.KiviArgs)
@@ -224,12 +239,14 @@ def _launch(q, kv, lengths, scale, split, n_splits, out, lse, tail=None) -> None
     if quant:
         ks, kz, vs, vz = grids
         for name, g in (("k_scale", ks), ("k_zero", kz), ("v_scale", vs), ("v_zero", vz)):
-            _require(g.dtype == torch.float16, f"{name} must be float16, got {g.dtype}")
-        _require(ks.dim() == 4 and ks.shape == kz.shape and tuple(ks.shape[:2]) == (b, hkv) and ks.shape[3] == d,
-                 f"k_scale / k_zero must be [{b}, {hkv}, groups, {d}]")
-        _require(ks.stride() == kz.stride() and ks.stride(-1) == 1, "k_scale and k_zero must share contiguous channels")
-        _require(tuple(vs.shape) == (b, hkv, t_max) and vs.shape == vz.shape and vs.stride() == vz.stride()
-                 and vs.stride(-1) == 1, f"v_scale / v_zero must be [{b}, {hkv}, {t_max}] with unit token stride")
+            if not (g.dtype == torch.float16):
+                raise ValueError(f"{name} must be float16, got {g.dtype}")
+        if not (ks.dim() == 4 and ks.shape == kz.shape and tuple(ks.shape[:2]) == (b, hkv) and ks.shape[3] == d):
+            raise ValueError(f"k_scale / k_zero must be [{b}, {hkv}, groups, {d}]")
+        if not (ks.stride() == kz.stride() and ks.stride(-1) == 1):
+            raise ValueError("k_scale and k_zero must share contiguous channels")
+        if not (tuple(vs.shape) == (b, hkv, t_max) and vs.shape == vz.shape and vs.stride() == vz.stride() and vs.stride(-1) == 1):
+            raise ValueError(f"v_scale / v_zero must be [{b}, {hkv}, {t_max}] with unit token stride")
         a.num_groups = ks.shape[2]
         a.k_scale, a.k_zero = ks.data_ptr(), kz.data_ptr()
         a.kgrid_stride_b, a.kgrid_stride_h, a.kgrid_stride_g = ks.stride(0), ks.stride(1), ks.stride(2)
@@ -242,23 +259,26 @@ def _launch(q, kv, lengths, scale, split, n_splits, out, lse, tail=None) -> None
     a.lse_stride_b, a.lse_stride_h, a.lse_stride_s = lse.stride(0), lse.stride(1), lse.stride(2)
     if tail is not None:
         tk, tv = tail
-        _require(tk.dim() == 4 and tk.shape == tv.shape and tuple(tk.shape[:2]) == (b, hkv) and tk.shape[3] == d,
-                 f"tail keys and values must be [{b}, {hkv}, tail_len, {d}]")
-        _require(tk.dtype == tv.dtype and tk.dtype in _Q_CODES, "tail keys and values must share a bf16/f16/f32 dtype")
-        _require(tk.stride() == tv.stride() and tk.stride(-1) == 1, "tail keys and values must share strides, channels contiguous")
-        _require(tk.device == dev and tv.device == dev, f"the tail must be on {dev}")
+        if not (tk.dim() == 4 and tk.shape == tv.shape and tuple(tk.shape[:2]) == (b, hkv) and tk.shape[3] == d):
+            raise ValueError(f"tail keys and values must be [{b}, {hkv}, tail_len, {d}]")
+        if not (tk.dtype == tv.dtype and tk.dtype in _Q_CODES):
+            raise ValueError("tail keys and values must share a bf16/f16/f32 dtype")
+        if not (tk.stride() == tv.stride() and tk.stride(-1) == 1):
+            raise ValueError("tail keys and values must share strides, channels contiguous")
+        if not (tk.device == dev and tv.device == dev):
+            raise ValueError(f"the tail must be on {dev}")
         a.tail_k, a.tail_v = tk.data_ptr(), tv.data_ptr()
         a.tail_stride_b, a.tail_stride_h, a.tail_stride_t = tk.stride(0), tk.stride(1), tk.stride(2)
         a.tail_dtype, a.tail_len = _Q_CODES[tk.dtype], tk.shape[2]
     lib = _lib.lib()
-    ws_bytes, cnt_bytes = ctypes.c_size_t(0), ctypes.c_size_t(0)
-    _lib.check(lib.bpt_kivi_plan(ctypes.byref(a), ctypes.byref(ws_bytes), ctypes.byref(cnt_bytes)))
-    stream = torch.cuda.current_stream(dev).cuda_stream
+    ws_bytes, cnt_bytes = ctypes.c_size_t(), ctypes.c_size_t()
+    _lib.check(lib.bpt_kivi_plan(a, ws_bytes, cnt_bytes))
+    stream = _stream(dev)
     workspace = cached_buffer("partials", dev, stream, ws_bytes.value)
     counters = cached_buffer("counters", dev, stream, cnt_bytes.value)
     a.workspace, a.workspace_bytes = workspace.data_ptr(), workspace.numel()
     a.counters, a.counters_bytes = counters.data_ptr(), counters.numel()
-    _lib.check(lib.bpt_kivi_decode(ctypes.byref(a), ctypes.c_void_p(stream)))
+    _lib.check(lib.bpt_kivi_decode(a, stream))
 
 
 def decode_attention(

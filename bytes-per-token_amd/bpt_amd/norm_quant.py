@@ -16,6 +16,7 @@ import torch
 
 from . import _lib
 from ._lib import F_BF16, F_F16, F_F32
+from .paged_attention import _stream
 
 _CODES = {torch.bfloat16: F_BF16, torch.float16: F_F16, torch.float32: F_F32}
 
@@ -59,6 +60,5 @@ def rms_norm_int8(
     a.weight = weight.data_ptr()
     a.codes, a.codes_stride_row = codes.data_ptr(), codes.stride(0)
     a.scale = scale.data_ptr()
-    stream = torch.cuda.current_stream(x.device).cuda_stream
-    _lib.check(_lib.lib().bpt_rms_norm_int8(ctypes.byref(a), ctypes.c_void_p(stream)))
+    _lib.check(_lib.lib().bpt_rms_norm_int8(a, _stream(x.device)))
     return codes.view(x.shape), scale.view(*x.shape[:-1], 1)

@@ -52,85 +52,84 @@ def kv_dtype_code(dtype: torch.dtype) -> int:
     raise ValueError(f"KV cache dtype must be bfloat16, float8_e4m3fn or int8, got {dtype}")
 
 
-def _ptr(t: torch.Tensor | None) -> int | None:
-    return None if t is None else t.data_ptr()
-
-
 def _stream(device: torch.device) -> int:
-    return torch.cuda.current_stream(device).cuda_stream
-
-
-def _require(cond: bool, msg: str) -> None:
-    if not cond:
-        raise ValueError(msg)
+    """The device's current HIP stream as an integer handle (without the object that torch.cuda.current_stream makes)."""
+    return torch._C._cuda_getCurrentRawStream(torch.cuda.current_device() if device.index is None else device.index)
 
 
 def _scale_layout(k_scale, v_scale, kv_code: int, pool_shape) -> tuple[int, tuple[int, int, int]]:
     """Scale kind and the (block, token, head) strides of per-token-head scale pools."""
     if kv_code == KV_BF16:
-        _require(k_scale is None and v_scale is None, "a bfloat16 cache takes no scales")
+        if not (k_scale is None and v_scale is None):
+            raise ValueError("a bfloat16 cache takes no scales")
         return SCALE_NONE, (0, 0, 0)
-    _require(k_scale is not None and v_scale is not None, "k_scale and v_scale are required for a quantized cache")
+    if not (k_scale is not None and v_scale is not None):
+        raise ValueError("k_scale and v_scale are required for a quantized cache")
     for s in (k_scale, v_scale):
-        _require(s.dtype == torch.float32, f"scales must be float32, got {s.dtype}")
+        if not (s.dtype == torch.float32):
+            raise ValueError(f"scales must be float32, got {s.dtype}")
     nb, p, hkv, _ = pool_shape
     if k_scale.dim() == 1:
-        _require(tuple(k_scale.shape) == (hkv,) and tuple(v_scale.shape) == (hkv,), f"per-head scales must be [{hkv}]")
-        _require(k_scale.is_contiguous() and v_scale.is_contiguous(), "per-head scales must be contiguous")
+        if not (tuple(k_scale.shape) == (hkv,) and tuple(v_scale.shape) == (hkv,)):
+            raise ValueError(f"per-head scales must be [{hkv}]")
+        if not (k_scale.is_contiguous() and v_scale.is_contiguous()):
+            raise ValueError("per-head scales must be contiguous")
         return SCALE_PER_HEAD, (0, 0, 0)
-    _require(
-        tuple(k_scale.shape) == (nb, p, hkv) and tuple(v_scale.shape) == (nb, p, hkv),
-        f"per-token-head scales must be [{nb}, {p}, {hkv}] like the pools",
-    )
-    _require(k_scale.stride() == v_scale.stride(), "k_scale and v_scale must share strides")
+    if not (tuple(k_scale.shape) == (nb, p, hkv) and tuple(v_scale.shape) == (nb, p, hkv)):
+        raise ValueError(f"per-token-head scales must be [{nb}, {p}, {hkv}] like the pools")
+    if not (k_scale.stride() == v_scale.stride()):
+        raise ValueError("k_scale and v_scale must share strides")
     return SCALE_PER_TOKEN_HEAD, tuple(k_scale.stride())
 
 
 def _decode_args(
     q, k_cache, v_cache, block_table, context_lens, k_scale, v_scale, scale, max_context, num_splits, out_dtype
 ) -> tuple[_lib.DecodeArgs, tuple[int, int, int, int]]:
-    _require(q.dim() == 4, f"q must be [B, Q, Hq, D], got {tuple(q.shape)}")
+    if not (q.dim() == 4):
+        raise ValueError(f"q must be [B, Q, Hq, D], got {tuple(q.shape)}")
     b, nq, hq, d = q.shape
-    _require(q.dtype in _FLOAT_CODES, f"q must be bf16, f16 or f32, got {q.dtype}")
-    _require(q.stride(-1) == 1, "q's channel dimension must be contiguous")
-    _require(k_cache.dim() == 4 and k_cache.shape == v_cache.shape, "k_cache and v_cache must be [NB, P, Hkv, D]")
-    _require(k_cache.dtype == v_cache.dtype, "k_cache and v_cache must share a dtype")
-    _require(k_cache.stride() == v_cache.stride(), "k_cache and v_cache must share strides")
-    _require(k_cache.stride(-1) == 1, "the caches' channel dimension must be contiguous")
+    if not (q.dtype in _FLOAT_CODES):
+        raise ValueError(f"q must be bf16, f16 or f32, got {q.dtype}")
+    if not (q.stride(-1) == 1):
+        raise ValueError("q's channel dimension must be contiguous")
+    if not (k_cache.dim() == 4 and k_cache.shape == v_cache.shape):
+        raise ValueError("k_cache and v_cache must be [NB, P, Hkv, D]")
+    if not (k_cache.dtype == v_cache.dtype):
+        raise ValueError("k_cache and v_cache must share a dtype")
+    if not (k_cache.stride() == v_cache.stride()):
+        raise ValueError("k_cache and v_cache must share strides")
+    if not (k_cache.stride(-1) == 1):
+        raise ValueError("the caches' channel dimension must be contiguous")
     kv_code = kv_dtype_code(k_cache.dtype)
     nb, page, hkv, dk = k_cache.shape
-    _require(dk == d, f"q head_dim {d} != cache head_dim {dk}")
-    _require(block_table.dim() == 2 and block_table.shape[0] == b, f"block_table must be [{b}, max_blocks]")
-    _require(block_table.dtype in _INDEX_CODES, "block_table must be int32 or int64")
-    _require(block_table.stride(1) == 1, "block_table rows must be contiguous")
+    if not (dk == d):
+        raise ValueError(f"q head_dim {d} != cache head_dim {dk}")
+    if not (block_table.dim() == 2 and block_table.shape[0] == b):
+        raise ValueError(f"block_table must be [{b}, max_blocks]")
+    if not (block_table.dtype in _INDEX_CODES):
+        raise ValueError("block_table must be int32 or int64")
+    if not (block_table.stride(1) == 1):
+        raise ValueError("block_table rows must be contiguous")
     if context_lens is not None:
-        _require(context_lens.dim() == 1 and context_lens.shape[0] == b, f"context_lens must be [{b}]")
-        _require(context_lens.dtype == torch.int32 and context_lens.is_contiguous(), "context_lens must be contiguous int32")
-    _require(out_dtype in _FLOAT_CODES, f"out dtype must be bf16, f16 or f32, got {out_dtype}")
+        if not (context_lens.dim() == 1 and context_lens.shape[0] == b):
+            raise ValueError(f"context_lens must be [{b}]")
+        if not (context_lens.dtype == torch.int32 and context_lens.is_contiguous()):
+            raise ValueError("context_lens must be contiguous int32")
+    if not (out_dtype in _FLOAT_CODES):
+        raise ValueError(f"out dtype must be bf16, f16 or f32, got {out_dtype}")
     scale_kind, sc_strides = _scale_layout(k_scale, v_scale, kv_code, k_cache.shape)
 
-    a = _lib.DecodeArgs()
-    a.struct_size = ctypes.sizeof(_lib.DecodeArgs)
-    a.kv_dtype = kv_code
-    a.scale_kind = scale_kind
-    a.q_dtype = _FLOAT_CODES[q.dtype]
-    a.out_dtype = _FLOAT_CODES[out_dtype]
-    a.table_dtype = _INDEX_CODES[block_table.dtype]
-    a.batch, a.num_queries, a.num_q_heads, a.num_kv_heads, a.head_dim, a.page_size = b, nq, hq, hkv, d, page
-    a.num_blocks = nb
-    a.max_blocks_per_seq = block_table.shape[1]
-    a.max_context = int(max_context)
-    a.num_splits = int(num_splits or 0)
-    a.sm_scale = float(scale)
-    a.q = q.data_ptr()
-    a.q_stride_b, a.q_stride_q, a.q_stride_h = q.stride(0), q.stride(1), q.stride(2)
-    a.k_cache, a.v_cache = k_cache.data_ptr(), v_cache.data_ptr()
-    a.kv_stride_block, a.kv_stride_token, a.kv_stride_head = k_cache.stride(0), k_cache.stride(1), k_cache.stride(2)
-    a.k_scale, a.v_scale = _ptr(k_scale), _ptr(v_scale)
-    a.scale_stride_block, a.scale_stride_token, a.scale_stride_head = sc_strides
-    a.block_table = block_table.data_ptr()
-    a.table_stride_b = block_table.stride(0)
-    a.context_lens = _ptr(context_lens)
+    q_sb, q_sq, q_sh, _ = q.stride()
+    kv_sb, kv_st, kv_sh, _ = k_cache.stride()
+    # The fields of bpt_decode_args in order, up to context_lens (one call: a field at a time costs twice as much).
+    a = _lib.DecodeArgs(
+        _lib.DECODE_ARGS_SIZE, kv_code, scale_kind, _FLOAT_CODES[q.dtype], _FLOAT_CODES[out_dtype],
+        _INDEX_CODES[block_table.dtype], b, nq, hq, hkv, d, page, nb, block_table.shape[1], int(max_context),
+        int(num_splits or 0), 0, 0, 0, float(scale), q.data_ptr(), q_sb, q_sq, q_sh, k_cache.data_ptr(),
+        v_cache.data_ptr(), kv_sb, kv_st, kv_sh, None if k_scale is None else k_scale.data_ptr(),
+        None if v_scale is None else v_scale.data_ptr(), *sc_strides, block_table.data_ptr(), block_table.stride(0),
+        None if context_lens is None else context_lens.data_ptr(),
+    )
     return a, (b, nq, hq, d)
 
 
@@ -174,7 +173,8 @@ _GRAIN = 1 << 20
 
 def cached_buffer(kind: str, device: torch.device, stream: int, nbytes: int) -> torch.Tensor:
     """The cached zero-initialized uint8 buffer `kind` for (device, stream), grown to at least `nbytes`."""
-    key = (kind, device.index if device.index is not None else torch.cuda.current_device(), stream)
+    index = device.index
+    key = (kind, torch.cuda.current_device() if index is None else index, stream)
     buf = _BUFFERS.get(key)
     if buf is None or buf.numel() < nbytes:
         size = max((nbytes + _GRAIN - 1) // _GRAIN * _GRAIN, _GRAIN)
@@ -230,21 +230,25 @@ def paged_decode_attention(
         out.dtype if out is not None else out_dtype,
     )
     dev = q.device
-    _require(dev.type == "cuda", "paged_decode_attention runs on a GPU: q must be a cuda tensor")
+    if dev.type != "cuda":
+        raise ValueError("paged_decode_attention runs on a GPU: q must be a cuda tensor")
     for name, t in (("k_cache", k_cache), ("v_cache", v_cache), ("block_table", block_table),
                     ("context_lens", context_lens), ("k_scale", k_scale), ("v_scale", v_scale)):
-        _require(t is None or t.device == dev, f"{name} is on {t.device if t is not None else None}, q on {dev}")
+        if t is not None and t.device != dev:
+            raise ValueError(f"{name} is on {t.device}, q on {dev}")
     if out is None:
         out4 = torch.empty((b, nq, hq, d), dtype=out_dtype, device=dev)
     else:
         out4 = out[:, None] if out.dim() == 3 else out
-        _require(tuple(out4.shape) == (b, nq, hq, d), f"out must be [{b}, {nq}, {hq}, {d}]")
-        _require(out4.stride(-1) == 1 and out4.device == dev, "out must be a cuda tensor with contiguous channels")
+        if not (tuple(out4.shape) == (b, nq, hq, d)):
+            raise ValueError(f"out must be [{b}, {nq}, {hq}, {d}]")
+        if not (out4.stride(-1) == 1 and out4.device == dev):
+            raise ValueError("out must be a cuda tensor with contiguous channels")
     a.out = out4.data_ptr()
-    a.out_stride_b, a.out_stride_q, a.out_stride_h = out4.stride(0), out4.stride(1), out4.stride(2)
+    a.out_stride_b, a.out_stride_q, a.out_stride_h, _ = out4.stride()
     if lse is not None:
-        _require(lse.dtype == torch.float32 and lse.is_contiguous() and lse.numel() == b * nq * hq and lse.device == dev,
-                 f"lse must be a contiguous float32 tensor of {b} x {nq} x {hq} on q's device")
+        if not (lse.dtype == torch.float32 and lse.is_contiguous() and lse.numel() == b * nq * hq and lse.device == dev):
+            raise ValueError(f"lse must be a contiguous float32 tensor of {b} x {nq} x {hq} on q's device")
         a.lse_out = lse.data_ptr()
     if _cascade is not None:  # the cascade's two launches (cascade.py): flags, length offset, partial to merge
         a.flags = _cascade.get("flags", 0)
@@ -252,30 +256,31 @@ def paged_decode_attention(
         merge = _cascade.get("merge")
         if merge is not None:
             m_out, m_lse = merge
-            _require(m_out.dtype == torch.float32 and m_out.is_contiguous() and tuple(m_out.shape) == (b, nq, hq, d),
-                     "the merged partial must be contiguous float32 [B, Q, Hq, D]")
-            _require(m_lse.dtype == torch.float32 and m_lse.is_contiguous() and m_lse.numel() == b * nq * hq,
-                     "the merged partial's lse must be contiguous float32 [B, Q, Hq]")
+            if not (m_out.dtype == torch.float32 and m_out.is_contiguous() and tuple(m_out.shape) == (b, nq, hq, d)):
+                raise ValueError("the merged partial must be contiguous float32 [B, Q, Hq, D]")
+            if not (m_lse.dtype == torch.float32 and m_lse.is_contiguous() and m_lse.numel() == b * nq * hq):
+                raise ValueError("the merged partial's lse must be contiguous float32 [B, Q, Hq]")
             a.merge_out, a.merge_lse = m_out.data_ptr(), m_lse.data_ptr()
     lib = _lib.lib()
-    ws_bytes, cnt_bytes = ctypes.c_size_t(0), ctypes.c_size_t(0)
-    _lib.check(lib.bpt_decode_plan(ctypes.byref(a), ctypes.byref(ws_bytes), ctypes.byref(cnt_bytes)))
     stream = _stream(dev)
-    if workspace is None:
-        workspace = cached_buffer("partials", dev, stream, ws_bytes.value)
-    if counters is None:
-        counters = cached_buffer("counters", dev, stream, cnt_bytes.value)
+    if workspace is None or counters is None:
+        ws_bytes, cnt_bytes = ctypes.c_size_t(), ctypes.c_size_t()
+        _lib.check(lib.bpt_decode_plan(a, ws_bytes, cnt_bytes))
+        if workspace is None:
+            workspace = cached_buffer("partials", dev, stream, ws_bytes.value)
+        if counters is None:
+            counters = cached_buffer("counters", dev, stream, cnt_bytes.value)
     for name, t in (("workspace", workspace), ("counters", counters)):
-        _require(t.device == dev and t.is_contiguous(), f"{name} must be a contiguous tensor on q's device")
-    a.workspace, a.workspace_bytes = workspace.data_ptr(), workspace.numel() * workspace.element_size()
-    a.counters, a.counters_bytes = counters.data_ptr(), counters.numel() * counters.element_size()
+        if t.device != dev or not t.is_contiguous():
+            raise ValueError(f"{name} must be a contiguous tensor on q's device")
+    a.workspace, a.workspace_bytes = workspace.data_ptr(), workspace.nbytes
+    a.counters, a.counters_bytes = counters.data_ptr(), counters.nbytes
     if _append is not None:  # paged_append_decode: store the new rows, then attend (one launch where it can)
-        _lib.check(lib.bpt_paged_append_decode(ctypes.byref(_append), ctypes.byref(a), ctypes.c_void_p(stream)))
+        _lib.check(lib.bpt_paged_append_decode(_append, a, stream))
     elif _events is None:
-        _lib.check(lib.bpt_paged_decode(ctypes.byref(a), ctypes.c_void_p(stream)))
+        _lib.check(lib.bpt_paged_decode(a, stream))
     else:  # measurement: two raw hipEvent_t handles recorded around the kernel itself
-        _lib.check(lib.bpt_paged_decode_timed(ctypes.byref(a), ctypes.c_void_p(stream), ctypes.c_void_p(_events[0]),
-                                              ctypes.c_void_p(_events[1])))
+        _lib.check(lib.bpt_paged_decode_timed(a, stream, _events[0], _events[1]))
     result = out if out is not None else out4
     return result[:, 0] if (squeeze and result.dim() == 4) else result
 
@@ -298,45 +303,51 @@ def quantize_append(
     BF16: the rows are copied. Rows whose page is negative or outside the pool are skipped.
     """
     a, dev = _append_args(k, v, k_cache, v_cache, k_scale, v_scale, write_blocks, write_offsets)
-    _lib.check(_lib.lib().bpt_quant_append(ctypes.byref(a), ctypes.c_void_p(_stream(dev))))
+    _lib.check(_lib.lib().bpt_quant_append(a, _stream(dev)))
 
 
 def _append_args(k, v, k_cache, v_cache, k_scale, v_scale, write_blocks, write_offsets):
     """The checked bpt_append_args of quantize_append's arguments, and their device."""
-    _require(k.dim() == 4 and k.shape == v.shape, "k and v must be [B, Q, Hkv, D]")
-    _require(k.dtype == v.dtype and k.dtype in _FLOAT_CODES, "k and v must share a bf16/f16/f32 dtype")
-    _require(k.stride() == v.stride() and k.stride(-1) == 1, "k and v must share strides, channels contiguous")
+    if not (k.dim() == 4 and k.shape == v.shape):
+        raise ValueError("k and v must be [B, Q, Hkv, D]")
+    if not (k.dtype == v.dtype and k.dtype in _FLOAT_CODES):
+        raise ValueError("k and v must share a bf16/f16/f32 dtype")
+    if not (k.stride() == v.stride() and k.stride(-1) == 1):
+        raise ValueError("k and v must share strides, channels contiguous")
     b, nq, hkv, d = k.shape
-    _require(k_cache.dim() == 4 and k_cache.shape == v_cache.shape, "k_cache and v_cache must be [NB, P, Hkv, D]")
-    _require(k_cache.dtype == v_cache.dtype and k_cache.stride() == v_cache.stride(), "caches must match")
-    _require(k_cache.shape[2] == hkv and k_cache.shape[3] == d, "cache heads/head_dim must match the rows")
-    _require(k_cache.stride(-1) == 1, "the caches' channel dimension must be contiguous")
+    if not (k_cache.dim() == 4 and k_cache.shape == v_cache.shape):
+        raise ValueError("k_cache and v_cache must be [NB, P, Hkv, D]")
+    if not (k_cache.dtype == v_cache.dtype and k_cache.stride() == v_cache.stride()):
+        raise ValueError("caches must match")
+    if not (k_cache.shape[2] == hkv and k_cache.shape[3] == d):
+        raise ValueError("cache heads/head_dim must match the rows")
+    if not (k_cache.stride(-1) == 1):
+        raise ValueError("the caches' channel dimension must be contiguous")
     kv_code = kv_dtype_code(k_cache.dtype)
     scale_kind, sc_strides = _scale_layout(k_scale, v_scale, kv_code, k_cache.shape)
-    _require(write_blocks.shape == (b, nq) and write_offsets.shape == (b, nq), f"write slots must be [{b}, {nq}]")
-    _require(write_blocks.dtype == write_offsets.dtype and write_blocks.dtype in _INDEX_CODES, "slots: int32/int64")
-    _require(write_blocks.stride() == write_offsets.stride(), "write_blocks and write_offsets must share strides")
+    if not (write_blocks.shape == (b, nq) and write_offsets.shape == (b, nq)):
+        raise ValueError(f"write slots must be [{b}, {nq}]")
+    if not (write_blocks.dtype == write_offsets.dtype and write_blocks.dtype in _INDEX_CODES):
+        raise ValueError("slots: int32/int64")
+    if not (write_blocks.stride() == write_offsets.stride()):
+        raise ValueError("write_blocks and write_offsets must share strides")
     dev = k.device
-    _require(dev.type == "cuda", "quantize_append runs on a GPU: k must be a cuda tensor")
+    if not (dev.type == "cuda"):
+        raise ValueError("quantize_append runs on a GPU: k must be a cuda tensor")
     for name, t in (("v", v), ("k_cache", k_cache), ("v_cache", v_cache), ("write_blocks", write_blocks),
                     ("write_offsets", write_offsets), ("k_scale", k_scale), ("v_scale", v_scale)):
-        _require(t is None or t.device == dev, f"{name} is not on {dev}")
+        if not (t is None or t.device == dev):
+            raise ValueError(f"{name} is not on {dev}")
 
-    a = _lib.AppendArgs()
-    a.struct_size = ctypes.sizeof(_lib.AppendArgs)
-    a.kv_dtype, a.scale_kind = kv_code, scale_kind
-    a.src_dtype = _FLOAT_CODES[k.dtype]
-    a.slot_dtype = _INDEX_CODES[write_blocks.dtype]
-    a.batch, a.num_queries, a.num_kv_heads, a.head_dim = b, nq, hkv, d
-    a.page_size, a.num_blocks = k_cache.shape[1], k_cache.shape[0]
-    a.k, a.v = k.data_ptr(), v.data_ptr()
-    a.new_stride_b, a.new_stride_q, a.new_stride_h = k.stride(0), k.stride(1), k.stride(2)
-    a.write_blocks, a.write_offsets = write_blocks.data_ptr(), write_offsets.data_ptr()
-    a.slot_stride_b, a.slot_stride_q = write_blocks.stride(0), write_blocks.stride(1)
-    a.k_cache, a.v_cache = k_cache.data_ptr(), v_cache.data_ptr()
-    a.kv_stride_block, a.kv_stride_token, a.kv_stride_head = k_cache.stride(0), k_cache.stride(1), k_cache.stride(2)
-    a.k_scale, a.v_scale = _ptr(k_scale), _ptr(v_scale)
-    a.scale_stride_block, a.scale_stride_token, a.scale_stride_head = sc_strides
+    n_sb, n_sq, n_sh, _ = k.stride()
+    kv_sb, kv_st, kv_sh, _ = k_cache.stride()
+    # The fields of bpt_append_args in order.
+    a = _lib.AppendArgs(
+        _lib.APPEND_ARGS_SIZE, kv_code, scale_kind, _FLOAT_CODES[k.dtype], _INDEX_CODES[write_blocks.dtype], b, nq, hkv,
+        d, k_cache.shape[1], k_cache.shape[0], k.data_ptr(), v.data_ptr(), n_sb, n_sq, n_sh, write_blocks.data_ptr(),
+        write_offsets.data_ptr(), *write_blocks.stride(), k_cache.data_ptr(), v_cache.data_ptr(), kv_sb, kv_st, kv_sh,
+        None if k_scale is None else k_scale.data_ptr(), None if v_scale is None else v_scale.data_ptr(), *sc_strides,
+    )
     return a, dev
 
 
@@ -370,7 +381,8 @@ def paged_append_decode(
     same results.
     """
     a, dev = _append_args(k, v, k_cache, v_cache, k_scale, v_scale, write_blocks, write_offsets)
-    _require(q.device == dev, f"q is on {q.device}, the new rows on {dev}")
+    if not (q.device == dev):
+        raise ValueError(f"q is on {q.device}, the new rows on {dev}")
     return paged_decode_attention(q, k_cache, v_cache, block_table, context_lens, k_scale, v_scale, scale=scale,
                                   max_context=max_context, num_splits=num_splits, out=out, out_dtype=out_dtype,
                                   _append=a)
@@ -393,20 +405,25 @@ def paged_prepare(
     [B, Q] and context_lens [B] (the last position + 1, clamped to the reserved tokens). A position gets a write
     block only when it is its row's token context_len - Q + i inside the reserved blocks (-1 otherwise: positions
     past the reservation or out of order store nothing). One launch, no host read."""
-    _require(table.dtype == torch.int32 and table.dim() == 2 and table.stride(1) == 1, "table: int32 [slots, blocks]")
-    _require(reserved.dtype == torch.int32 and reserved.is_contiguous() and reserved.numel() == table.shape[0],
-             "reserved: int32 [slots]")
-    _require(positions.dim() == 2 and positions.dtype in _INDEX_CODES, "positions: int32 / int64 [B, Q]")
+    if not (table.dtype == torch.int32 and table.dim() == 2 and table.stride(1) == 1):
+        raise ValueError("table: int32 [slots, blocks]")
+    if not (reserved.dtype == torch.int32 and reserved.is_contiguous() and reserved.numel() == table.shape[0]):
+        raise ValueError("reserved: int32 [slots]")
+    if not (positions.dim() == 2 and positions.dtype in _INDEX_CODES):
+        raise ValueError("positions: int32 / int64 [B, Q]")
     b, nq = positions.shape
-    _require(slots.dtype == torch.int32 and slots.is_contiguous() and slots.numel() == b, f"slots: int32 [{b}]")
+    if not (slots.dtype == torch.int32 and slots.is_contiguous() and slots.numel() == b):
+        raise ValueError(f"slots: int32 [{b}]")
     for name, t, shape in (("block_table", block_table, None), ("write_blocks", write_blocks, (b, nq)),
                            ("write_offsets", write_offsets, (b, nq)), ("context_lens", context_lens, (b,))):
-        _require(t.dtype == torch.int32 and t.is_contiguous() and (shape is None or tuple(t.shape) == shape),
-                 f"{name}: contiguous int32")
-    _require(block_table.dim() == 2 and block_table.shape[0] == b, f"block_table: [{b}, n_blocks]")
+        if not (t.dtype == torch.int32 and t.is_contiguous() and (shape is None or tuple(t.shape) == shape)):
+            raise ValueError(f"{name}: contiguous int32")
+    if not (block_table.dim() == 2 and block_table.shape[0] == b):
+        raise ValueError(f"block_table: [{b}, n_blocks]")
     dev = positions.device
     for name, t in (("table", table), ("reserved", reserved), ("slots", slots), ("block_table", block_table)):
-        _require(t.device == dev, f"{name} is not on {dev}")
+        if not (t.device == dev):
+            raise ValueError(f"{name} is not on {dev}")
     a = _lib.PrepareArgs()
     a.struct_size = ctypes.sizeof(_lib.PrepareArgs)
     a.batch, a.num_queries, a.n_blocks = b, nq, block_table.shape[1]
@@ -417,7 +434,7 @@ def paged_prepare(
     a.positions, a.pos_stride_b, a.pos_stride_q = positions.data_ptr(), positions.stride(0), positions.stride(1)
     a.block_table, a.write_blocks = block_table.data_ptr(), write_blocks.data_ptr()
     a.write_offsets, a.context_lens = write_offsets.data_ptr(), context_lens.data_ptr()
-    _lib.check(_lib.lib().bpt_paged_prepare(ctypes.byref(a), ctypes.c_void_p(_stream(dev))))
+    _lib.check(_lib.lib().bpt_paged_prepare(a, _stream(dev)))
 
 
 def kv_read_bytes(context_lens_host, num_kv_heads: int, head_dim: int, kv_dtype: torch.dtype, per_token_scales: bool,
