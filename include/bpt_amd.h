@@ -111,7 +111,7 @@ typedef struct {
   int32_t chunk_tokens; /* out of bpt_decode_plan: tokens one wave streams per step */
   int32_t grid_groups;  /* out of bpt_decode_plan: workgroups launched */
   int32_t rows_per_group; /* out of bpt_decode_plan: query rows computed together per KV head; 16 = the
-                             matrix-core kernel (FP8 caches, 2..16 rows; INT8, 5..16), 32/64/128 = the many-row
+                             matrix-core kernel (FP8 caches, 2..16 rows; INT8, 5..16), 32..256 = the many-row
                              matrix-core kernel (more than 16 rows), 1/2/4 = the vector kernel */
   float sm_scale;
 
