@@ -2,10 +2,11 @@
 
 When sequences start with the same pages (a system prompt, or the branches of a speculative verify step;
 fastserve's prefix cache decides the sharing, kv/prefix_cache.py:42-140), plain paged decode reads the
-shared pages once per sequence. The cascade reads them once per 16 query rows of the whole group:
+shared pages once per sequence. The cascade reads them once per 16 query rows of the whole group, or once per
+128 or 256 of them where the group's rows and the prefix are many (_one_sequence):
 
 1. Prefix pass. All queries of a group (members x Q queries x G heads per KV head) attend the group's
-   `prefix_pages` shared pages, 16 rows at a time, non-causally (every query sits after the prefix), and
+   `prefix_pages` shared pages, a group of rows at a time, non-causally (every query sits after the prefix), and
    leave float32 partials: each row's normalized output and log-sum-exp.
 2. Suffix pass. Every sequence attends its own pages after the prefix with the usual causal rule; each row's
    result is merged with its prefix partial as kernels/reference.py:205-211 merges split partials, so the
@@ -37,6 +38,18 @@ def _rows_per_pass(total_queries: int, heads_per_kv: int) -> int:
         if total_queries % qv == 0:
             best = qv
     return best
+
+
+def _one_sequence(rows: int, prefix: int, q_dtype: torch.dtype, kv_dtype: torch.dtype) -> bool:
+    """Whether the prefix pass takes all of a group's rows (queries times query heads per KV head) as one sequence, on
+    the many-row kernel: more than 16 rows of a bf16 or f16 q, and rows x prefix tokens large.
+
+    Measured, groups of 16 rows against one sequence, 8 KV heads (us): BF16 caches (whose groups are computed 4 rows at
+    a time) 20 rows x 512 tokens 15 : 20, 48 x 4096 54 : 24, 64 x 8192 101 : 30; FP8 64 x 8192 22 : 28, 512 x 1024
+    17 : 27, 256 x 16384 79 : 61; INT8 128 x 8192 39 : 36.
+    """
+    enough = 1 << 16 if kv_dtype == torch.bfloat16 else 1 << 20
+    return rows > 16 and q_dtype != torch.float32 and rows * prefix >= enough
 
 
 def cascade_decode_attention(
@@ -97,7 +110,8 @@ def cascade_decode_attention(
     part_lse = torch.empty((b, nq, hq), dtype=torch.float32, device=dev)
     for s, e in groups:
         total = (e - s) * nq
-        qv = _rows_per_pass(total, heads_per_kv)
+        whole = _one_sequence(total * heads_per_kv, prefix, q4.dtype, k_cache.dtype)
+        qv = total if whole else _rows_per_pass(total, heads_per_kv)
         nv = total // qv
         table = block_table[s, :prefix_pages].expand(nv, prefix_pages)
         paged_decode_attention(

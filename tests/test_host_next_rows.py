@@ -101,6 +101,14 @@ def test_norm_quant_needs_gpu_tensors():
         rms_norm_int8(torch.zeros(2, 8), torch.ones(4), 1e-6)
 
 
+def test_cascade_prefix_as_one_sequence():
+    bf, f8 = torch.bfloat16, torch.float8_e4m3fn
+    assert cascade._one_sequence(32, 2048, bf, bf) and not cascade._one_sequence(32, 2047, bf, bf)
+    assert cascade._one_sequence(512, 2048, torch.float16, f8) and not cascade._one_sequence(512, 2047, bf, f8)
+    assert not cascade._one_sequence(512, 8192, torch.float32, bf)  # an f32 q keeps float32 products
+    assert not cascade._one_sequence(16, 1 << 20, bf, f8)
+
+
 def test_cascade_rows_per_pass():
     assert cascade._rows_per_pass(80, 2) == 8  # 16 sequences x 5 queries, 2 heads per KV head: 10 passes of 16 rows
     assert cascade._rows_per_pass(15, 2) == 5
