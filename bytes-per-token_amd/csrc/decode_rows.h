@@ -14,8 +14,10 @@
 //    holds row n's scores of tokens 8 a + 4 hf + b (a, b < 4) of each 32; the second product's contraction index
 //    is mapped to exactly those tokens, so P^T is built in registers. V^T holds every 16 tokens in that order.
 // The codes are exact in 16 bits (FP8 and INT8 in bf16 and f16, BF16 as it is). The weights are float32 numbers
-// fed to the MFMAs as f16 plus f16 remainder (FP8 / INT8 values, 22 bits) or as three bf16 parts (BF16 values, 24
-// bits); an f16 q over a BF16 cache as bf16 plus bf16 remainder (exact).
+// fed to the MFMAs as the vector kernel takes them: over BF16 and INT8 values whole, as three bf16 parts (24 bits, the
+// range of float32: a per-token INT8 scale rides in them), over FP8 values as f16 plus f16 remainder (22 bits); an f16 q
+// over a BF16 cache as bf16 plus bf16 remainder (exact). (INT8 in two f16 parts is faster, 512 new over 8192 cached tokens,
+// 32 heads 154 us against 172, but drops bits that the vector kernel keeps, and scales past 2^64.)
 //
 // What bounds it: with many chunks the matrix cores (FP8: three products where two would do, for the weights' second
 // part) and the vector units behind them (256-row tiles, 2048 rows x 8 heads over 4096 tokens: 37 % and 52 % of the
@@ -58,6 +60,8 @@ struct RowsCfg {
   static constexpr bool kF16K = QF16_ && !kBf16;   // K and q operands in f16 (an f16 q over codes), else bf16
   static constexpr bool kQSplit = QF16_ && kBf16;  // an f16 q as two bf16 parts
   static constexpr bool kQF16 = QF16_;
+  static constexpr bool kVF16 = KV == kKvFp8;      // values and weights in f16 (weights in two parts), else bf16 (three)
+  static constexpr bool kVBound = kVF16 && SK == kScaleTokenHead;  // the reference point tracks vscale_bound
   static constexpr int kQOps = kQSplit ? 16 : 8;
   static constexpr int kGroups = CT / 16 / NW;     // 16-token groups a wave loads per chunk
   static constexpr int kKLoads = kBf16 ? 4 : 2;    // 16-byte K loads per group
@@ -217,9 +221,10 @@ __device__ __forceinline__ void rows_issue(const DecodeParams& p, int b, int h, 
   }
 }
 
-// Per-token scales of one chunk in LDS: K scales (times sm_scale log2 e), V scales, and vscale_bound of the latter.
+// Per-token scales of one chunk in LDS: K scales (times sm_scale log2 e), V scales, and (f16 weights) vscale_bound of
+// the latter.
 template <typename C>
-using RowsScales = float[3][C::SK == kScaleTokenHead ? C::CT : 1];
+using RowsScales = float[C::kVBound ? 3 : 2][C::SK == kScaleTokenHead ? C::CT : 1];
 
 template <typename C>
 __device__ __forceinline__ void rows_store(const DecodeParams& p, const RowsStage<C>& s, uint8_t* buf,
@@ -267,7 +272,7 @@ __device__ __forceinline__ void rows_store(const DecodeParams& p, const RowsStag
 #pragma unroll
       for (int i = 0; i < 8; ++i)
         *(u32x2*)(vrow + i * 128 + 16 * (unit ^ ((i + cl) & 7))) =
-            C::KV == kKvFp8 ? rows_fp8_to_f16(o[i]) : rows_int8_to_f16(o[i]);
+            C::KV == kKvFp8 ? rows_fp8_to_f16(o[i]) : rows_int8_to_bf16(o[i]);
     }
   }
   if constexpr (C::SK == kScaleTokenHead) {
@@ -275,7 +280,7 @@ __device__ __forceinline__ void rows_store(const DecodeParams& p, const RowsStag
       ssc[0][tid] = s.sc * p.qscale;
     } else if (tid < 2 * C::CT) {
       ssc[1][tid - C::CT] = s.sc;
-      ssc[2][tid - C::CT] = vscale_bound(s.sc);
+      if constexpr (C::kVBound) ssc[2][tid - C::CT] = vscale_bound(s.sc);
     }
   }
 }
@@ -291,7 +296,7 @@ __device__ __forceinline__ f32x16 rows_mfma_k(u32x4 a, u32x4 q, f32x16 acc) {
 }
 template <typename C>
 __device__ __forceinline__ f32x16 rows_mfma_v(u32x4 a, u32x4 w, f32x16 acc) {
-  if constexpr (C::kBf16)
+  if constexpr (!C::kVF16)
     return __builtin_amdgcn_mfma_f32_32x32x16_bf16(__builtin_bit_cast(bf16x8, a), __builtin_bit_cast(bf16x8, w), acc, 0, 0, 0);
   else
     return __builtin_amdgcn_mfma_f32_32x32x16_f16(__builtin_bit_cast(f16x8, a), __builtin_bit_cast(f16x8, w), acc, 0, 0, 0);
@@ -386,7 +391,7 @@ __device__ __forceinline__ void rows_compute(const uint8_t* buf, const RowsScale
       }
       mul = 1.0f;
     }
-    if constexpr (C::SK == kScaleTokenHead) {
+    if constexpr (C::kVBound) {
 #pragma unroll
       for (int a = 0; a < 4; ++a) {
         const f32x4 vb = *(const f32x4*)&ssc[2][th + 8 * a + 4 * hf];
@@ -430,7 +435,7 @@ __device__ __forceinline__ void rows_compute(const uint8_t* buf, const RowsScale
         }
       }
       u32x4 part[3];
-      if constexpr (C::kBf16) {
+      if constexpr (!C::kVF16) {
 #pragma unroll
         for (int q = 0; q < 3; ++q) {
 #pragma unroll
@@ -451,7 +456,7 @@ __device__ __forceinline__ void rows_compute(const uint8_t* buf, const RowsScale
         }
       }
 #pragma unroll
-      for (int q = 0; q < (C::kBf16 ? 3 : 2); ++q) {
+      for (int q = 0; q < (C::kVF16 ? 2 : 3); ++q) {
 #pragma unroll
         for (int ct = 0; ct < 4; ++ct) st.o[ct] = rows_mfma_v<C>(va[h2][ct], part[q], st.o[ct]);
       }

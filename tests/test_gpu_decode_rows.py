@@ -109,3 +109,37 @@ def test_rows_negative_scale_and_lse_and_repeats():
     seen = np.isfinite(want_lse)
     assert np.array_equal(np.isfinite(lse.cpu().numpy()), seen)
     assert np.abs(lse.cpu().numpy() - want_lse)[seen].max() < 1e-4
+
+
+@pytest.mark.parametrize("q_dtype", [torch.bfloat16, torch.float16])
+@pytest.mark.parametrize("hq,nq", [(17, 1), (33, 1), (65, 1), (300, 1), (64, 40)])
+def test_rows_int8_weights_keep_all_24_bits(hq, nq, q_dtype):
+    """One visible token with zero keys: its weight is 2^4 times its float32 value scale, so a code that is a power of two
+    gives that scale times the code exactly, if the weight keeps its 24 bits and its exponent (2^-60 .. 2^90)."""
+    from bpt_amd import paged_decode_attention
+
+    g = torch.Generator(device=DEV).manual_seed(hq)
+    b, t, hkv = 40, nq, 1
+    k = torch.zeros((b, 16 * 4, hkv, 128), dtype=torch.int8, device=DEV).view(b * 4, 16, hkv, 128)
+    codes = torch.tensor([1, 2, -4, 64, -128], dtype=torch.int8, device=DEV)
+    v = codes[torch.randint(5, k.shape, generator=g, device=DEV)]
+    vs = (torch.rand(k.shape[:3], generator=g, device=DEV) + 1) * torch.exp2(torch.randint(-60, 91, k.shape[:3], generator=g, device=DEV).float())
+    ks = torch.ones_like(vs)
+    table = torch.arange(b * 4, dtype=torch.int32, device=DEV).view(b, 4)
+    lens = torch.full((b,), t, dtype=torch.int32, device=DEV)
+    q = torch.randn((b, nq, hq, 128), generator=g, device=DEV).to(q_dtype)
+    got = paged_decode_attention(q, k, v, table, lens, ks, vs, scale=0.1, max_context=t, out_dtype=torch.float32)
+    want = v.view(b, 64, 128)[:, 0].float() * vs.view(b, 64)[:, :1]
+    assert torch.equal(got[:, 0], want[:, None].expand(b, hq, 128))  # the first query sees the first token alone
+
+
+def test_rows_int8_scales_over_the_float32_range():
+    """Value scales of 0 and from 2^-40 to 2^80 in one sequence, against the oracle: float32 within 2^-14 of the largest."""
+    c = make_case("int8", [700, 90], hq=64, hkv=2, nq=2, scales="token", seed=3)
+    g = torch.Generator(device=DEV).manual_seed(4)
+    for lo, hi in ((70, 81), (-40, -29), (-40, 81)):
+        e = torch.randint(lo, hi, c["vs"].shape, generator=g, device=DEV).float()
+        d = dict(c, vs=torch.where(torch.rand(e.shape, generator=g, device=DEV) < 0.2, 0.0, c["vs"] * torch.exp2(e)))
+        got, want = run_case(d, out_dtype=torch.float32)
+        err = np.abs(got.cpu().numpy() - want).max()
+        assert err <= 2.0**-14 * np.abs(want).max(), f"2^{lo} .. 2^{hi}: {err:.3e}"
