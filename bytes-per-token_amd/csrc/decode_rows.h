@@ -32,6 +32,13 @@
 //  * V: 64-token blocks of [channel][8 units], unit u of channel c at u ^ ((c + c / 8) % 8); unit 2 s + hf holds
 //    tokens 16 s + 4 hf + 0..3 and 16 s + 8 + 4 hf + 0..3. Reads take one unit of 8 consecutive channels; an 8-byte
 //    store takes one half unit of channels c, c + 8, ...: lanes of the upper 64 channels hold the other half.
+//
+// A token that a row does not see must add nothing to it, and the split weights must not turn an infinity into NaN, but
+// the MFMAs multiply every value by every weight and by every part of it, zeros included. So values that are not finite
+// (and per-token value scales that are not) are replaced by zeros on their way into LDS, and the rows that see them get
+// them added one by one (rows_add_nonfinite), which finite data never pays for; the look at the values costs BF16 caches
+// 1 to 2 % (2048 + 2048 tokens, 16 heads 132.5 -> 134.2 us, 512 + 8192, 32 heads 170 -> 171, with an f16 q 187 -> 192) and
+// the others nothing that shows (FP8 111 -> 110).
 #pragma once
 
 #include <type_traits>
@@ -46,6 +53,7 @@ typedef float f32x4 __attribute__((ext_vector_type(4)));
 typedef float f32x16 __attribute__((ext_vector_type(16)));
 typedef uint32_t u32x2 __attribute__((ext_vector_type(2)));
 typedef uint32_t u32x4 __attribute__((ext_vector_type(4)));
+typedef uint16_t u16x2 __attribute__((ext_vector_type(2)));
 
 template <int KV_, int SK_, bool PU_, bool QF16_, int WM_, int NW_, int NBUF_>
 struct RowsCfg {
@@ -61,6 +69,8 @@ struct RowsCfg {
   static constexpr bool kQSplit = QF16_ && kBf16;  // an f16 q as two bf16 parts
   static constexpr bool kQF16 = QF16_;
   static constexpr bool kVF16 = KV == kKvFp8;      // values and weights in f16 (weights in two parts), else bf16 (three)
+  // Whether values or value scales can be infinite or NaN (INT8 codes cannot).
+  static constexpr bool kNonfinite = KV != kKvInt8 || SK == kScaleTokenHead;
   static constexpr bool kVBound = kVF16 && SK == kScaleTokenHead;  // the reference point tracks vscale_bound
   static constexpr int kQOps = kQSplit ? 16 : 8;
   static constexpr int kGroups = CT / 16 / NW;     // 16-token groups a wave loads per chunk
@@ -226,9 +236,14 @@ __device__ __forceinline__ void rows_issue(const DecodeParams& p, int b, int h, 
 template <typename C>
 using RowsScales = float[C::kVBound ? 3 : 2][C::SK == kScaleTokenHead ? C::CT : 1];
 
+__device__ __forceinline__ bool rows_finite(float x) { return fabsf(x) <= __FLT_MAX__; }
+
+// Chunk kk's codes and scales into LDS. partial: some row of the tile does not see all of its tokens. *bad becomes
+// kk + 1 if values or value scales are not finite and were replaced by zeros: any of a BF16 chunk (whose infinities the
+// split weights would turn into NaN), NaN codes of a partial FP8 chunk (in the others every row gets the NaN anyway).
 template <typename C>
 __device__ __forceinline__ void rows_store(const DecodeParams& p, const RowsStage<C>& s, uint8_t* buf,
-                                           RowsScales<C>& ssc, int wave, int lane, int tid) {
+                                           RowsScales<C>& ssc, int kk, bool partial, int* bad, int wave, int lane, int tid) {
   uint8_t* kbuf = buf;
   uint8_t* vbuf = buf + C::CT * kHeadDim * 2;
 #pragma unroll
@@ -254,10 +269,23 @@ __device__ __forceinline__ void rows_store(const DecodeParams& p, const RowsStag
     const int unit = 2 * ((t0 & 63) >> 4) + (quad & 1);
     uint8_t* vrow = vbuf + (t0 >> 6) * 16384 + 8 * cl * 128 + 8 * (quad >> 1);
     if constexpr (C::kBf16) {
-      const uint32_t w[4][4] = {{s.v[u][0].x, s.v[u][0].y, s.v[u][0].z, s.v[u][0].w},
-                                {s.v[u][1].x, s.v[u][1].y, s.v[u][1].z, s.v[u][1].w},
-                                {s.v[u][2].x, s.v[u][2].y, s.v[u][2].z, s.v[u][2].w},
-                                {s.v[u][3].x, s.v[u][3].y, s.v[u][3].z, s.v[u][3].w}};
+      uint32_t w[4][4] = {{s.v[u][0].x, s.v[u][0].y, s.v[u][0].z, s.v[u][0].w},
+                          {s.v[u][1].x, s.v[u][1].y, s.v[u][1].z, s.v[u][1].w},
+                          {s.v[u][2].x, s.v[u][2].y, s.v[u][2].z, s.v[u][2].w},
+                          {s.v[u][3].x, s.v[u][3].y, s.v[u][3].z, s.v[u][3].w}};
+      u16x2 top = {0, 0};
+#pragma unroll
+      for (int i = 0; i < 16; ++i)
+        top = __builtin_elementwise_max(top, __builtin_bit_cast(u16x2, w[i >> 2][i & 3] & 0x7fff7fffu));
+      if (__any(top.x >= 0x7f80 || top.y >= 0x7f80)) {
+        *bad = kk + 1;
+#pragma unroll
+        for (int i = 0; i < 16; ++i) {
+          uint32_t& x = w[i >> 2][i & 3];
+          if ((x & 0x7f80u) == 0x7f80u) x &= 0xffff0000u;
+          if ((x & 0x7f800000u) == 0x7f800000u) x &= 0xffffu;
+        }
+      }
 #pragma unroll
       for (int i = 0; i < 8; ++i) {
         const uint32_t sel = (i & 1) ? 0x07060302u : 0x05040100u;
@@ -269,6 +297,18 @@ __device__ __forceinline__ void rows_store(const DecodeParams& p, const RowsStag
       uint32_t o[8];
       rows_transpose4(s.v[u][0].x, s.v[u][1].x, s.v[u][2].x, s.v[u][3].x, o);
       rows_transpose4(s.v[u][0].y, s.v[u][1].y, s.v[u][2].y, s.v[u][3].y, o + 4);
+      if constexpr (C::KV == kKvFp8) {
+        if (partial) {
+          uint32_t any = 0u;
+#pragma unroll
+          for (int i = 0; i < 8; ++i) {  // NaN: the code 0x7f with either sign
+            const uint32_t nan = ((o[i] & 0x7f7f7f7fu) + 0x01010101u) & 0x80808080u;
+            any |= nan;
+            o[i] &= ~((nan >> 7) * 0xffu);
+          }
+          if (__any(any != 0u)) *bad = kk + 1;
+        }
+      }
 #pragma unroll
       for (int i = 0; i < 8; ++i)
         *(u32x2*)(vrow + i * 128 + 16 * (unit ^ ((i + cl) & 7))) =
@@ -279,7 +319,9 @@ __device__ __forceinline__ void rows_store(const DecodeParams& p, const RowsStag
     if (tid < C::CT) {
       ssc[0][tid] = s.sc * p.qscale;
     } else if (tid < 2 * C::CT) {
-      ssc[1][tid - C::CT] = s.sc;
+      const bool fin = rows_finite(s.sc);
+      if (!fin) *bad = kk + 1;
+      ssc[1][tid - C::CT] = fin ? s.sc : 0.0f;
       if constexpr (C::kVBound) ssc[2][tid - C::CT] = vscale_bound(s.sc);
     }
   }
@@ -464,6 +506,53 @@ __device__ __forceinline__ void rows_compute(const uint8_t* buf, const RowsScale
     }
     st.l += l0 + l1;
     s = s_next;
+  }
+}
+
+// The values of tokens T .. T + n - 1 that rows_store replaced by zeros, added for the rows that see them.
+template <typename C>
+__device__ __forceinline__ void rows_add_nonfinite(const DecodeParams& p, int b, int h, int T, int n, int lane, int rlen,
+                                                   RowsState& st) {
+  const int32_t* table = (const int32_t*)p.table;
+  const int hf = lane >> 5;
+#pragma unroll 1
+  for (int tok = T; tok < T + n; ++tok) {
+    const int e = rows_clamp_page(p, load_uniform(table + table_word(p, b, tok >> p.logP)));
+    const int64_t in_page = tok & (p.P - 1);
+    const uint8_t* src = p.v + (int64_t)e * p.kv_sblk + in_page * p.kv_stok + (int64_t)h * p.kv_shead;
+    float mul = 1.0f;
+    if constexpr (C::SK == kScaleTokenHead) {
+      const float sc = p.vs[(int64_t)e * p.sc_sblk + in_page * p.sc_stok + (int64_t)h * p.sc_shead];
+      if (!rows_finite(sc)) mul = sc;
+    }
+#pragma unroll
+    for (int ct = 0; ct < 4; ++ct) {
+#pragma unroll
+      for (int a = 0; a < 4; ++a) {
+        const int ch = 32 * ct + 8 * a + 4 * hf;
+        float x[4];
+        if constexpr (C::kBf16) {
+          const u32x2 w = *(const u32x2*)(src + 2 * ch);
+          x[0] = __uint_as_float(w.x << 16);
+          x[1] = __uint_as_float(w.x & 0xffff0000u);
+          x[2] = __uint_as_float(w.y << 16);
+          x[3] = __uint_as_float(w.y & 0xffff0000u);
+        } else {
+          const uint32_t w = *(const uint32_t*)(src + ch);
+          if constexpr (C::KV == kKvFp8) {
+            fp8x4_to_f32(w, x);
+          } else {
+#pragma unroll
+            for (int j = 0; j < 4; ++j) x[j] = (float)(int8_t)((w >> (8 * j)) & 0xffu);
+          }
+        }
+#pragma unroll
+        for (int j = 0; j < 4; ++j) {
+          const float v = x[j] * mul;
+          if (tok < rlen && !rows_finite(v)) st.o[ct][4 * a + j] += v;
+        }
+      }
+    }
   }
 }
 
@@ -655,7 +744,7 @@ __global__ __launch_bounds__(kCombineWaves * 64) void rows_combine_kernel(const 
       f32x4 ov[kJ];
 #pragma unroll
       for (int j = 0; j < kJ; ++j) {
-        const int jj = min(j0 + j, n - 1);  // a piece past the last is read again and weighs nothing
+        const int jj = min(j0 + j, n - 1);  // a piece past the last is read again, for nothing
         const int64_t row = (2 * (g_first + jj) + (jj == 0 ? 1 : 0)) * BM + r;
         lv[j] = p.ws_lse[row];
         ov[j] = *(const f32x4*)(p.ws_out + row * D + ch);
@@ -663,7 +752,10 @@ __global__ __launch_bounds__(kCombineWaves * 64) void rows_combine_kernel(const 
       float nm = M;
 #pragma unroll
       for (int j = 0; j < kJ; ++j) {
-        if (j0 + j >= n) lv[j] = kNegInf;
+        if (j0 + j >= n) {
+          lv[j] = kNegInf;
+          ov[j] = f32x4{0.0f, 0.0f, 0.0f, 0.0f};
+        }
         nm = fmaxf(nm, lv[j]);
       }
       const float mu = nm == kNegInf ? 0.0f : nm;
@@ -695,6 +787,7 @@ __global__ __launch_bounds__(NW * 64, 2) void decode_rows_kernel(const DecodePar
   __shared__ int s_last;
   __shared__ __attribute__((aligned(16))) uint8_t smem[C::kSmem];
   __shared__ __attribute__((aligned(16))) RowsScales<C> s_sc[NBUF];
+  __shared__ int s_bad[NBUF];  // rows_store: 1 + the chunk in the buffer, if it holds values that are not finite
 
   const int tid = threadIdx.x;
   const int lane = tid & 63;
@@ -704,6 +797,7 @@ __global__ __launch_bounds__(NW * 64, 2) void decode_rows_kernel(const DecodePar
   const int rows = p.Q * p.G;
   int* s_len = s_dyn + B * T + 1;
 
+  if (tid < NBUF) s_bad[tid] = 0;
   build_tile_line<NW, BM>(p, s_line, s_len, s_wsum);
   // Sequences with no tokens: zero rows, or the caller's partial.
   for (int b = blockIdx.x; b < B; b += gridDim.x) {
@@ -773,6 +867,9 @@ __global__ __launch_bounds__(NW * 64, 2) void decode_rows_kernel(const DecodePar
     const int rlen_min = sread(rlen);  // lane 0's row sees the fewest tokens, the last lane's the most
     const int rlen_max = __builtin_amdgcn_readlane(rlen, 31);
 
+    // Chunks from this one on are not seen whole by the tile's first row.
+    const int partial = (p.noncausal ? len : max(len - (p.Q - 1 - t * BM / p.G), 0)) / C::CT;
+
     // The next piece of the range, if it holds chunks of one.
     int nb_ = b, nh = h, nt = t + 1, n_end = 0, nlen = 0, nspan = 0;
     int64_t nc0 = c0 + span;
@@ -804,7 +901,7 @@ __global__ __launch_bounds__(NW * 64, 2) void decode_rows_kernel(const DecodePar
 
     int cur = 0;
     if constexpr (NBUF == 2) {
-      rows_store<C>(p, stage, smem, s_sc[0], wave, lane, tid);
+      rows_store<C>(p, stage, smem, s_sc[0], k, k >= partial, s_bad, wave, lane, tid);
       __syncthreads();
     }
     for (int kk = k; kk < k_end; ++kk) {
@@ -814,7 +911,7 @@ __global__ __launch_bounds__(NW * 64, 2) void decode_rows_kernel(const DecodePar
       __asm__ volatile("" : "+v"(ln));
       if constexpr (NBUF == 1) {
         if (kk > k) __syncthreads();  // every wave is done with the previous chunk
-        rows_store<C>(p, stage, smem, s_sc[0], wave, ln, tid);
+        rows_store<C>(p, stage, smem, s_sc[0], kk, kk >= partial, s_bad, wave, ln, tid);
         __syncthreads();
       }
       const bool last = kk + 1 == k_end;
@@ -829,12 +926,16 @@ __global__ __launch_bounds__(NW * 64, 2) void decode_rows_kernel(const DecodePar
       {
         const int t0 = wn * C::TW;
         const int tok = kk * C::CT + t0;
-        if (tok < rlen_max) rows_compute<C>(smem + cur * C::kBuf, s_sc[cur], t0, tok, ln, qb, fabsf(qscale), rlen, rlen_min, st);
+        if (tok < rlen_max) {
+          rows_compute<C>(smem + cur * C::kBuf, s_sc[cur], t0, tok, ln, qb, fabsf(qscale), rlen, rlen_min, st);
+          if (C::kNonfinite && sread(s_bad[cur]) == kk + 1)
+            rows_add_nonfinite<C>(p, b, h, tok, min(C::TW, rlen_max - tok), ln, rlen, st);
+        }
       }
       if constexpr (NBUF == 2) {
         if (!last) {
           cur ^= 1;
-          rows_store<C>(p, stage, smem + cur * C::kBuf, s_sc[cur], wave, ln, tid);
+          rows_store<C>(p, stage, smem + cur * C::kBuf, s_sc[cur], kk + 1, kk + 1 >= partial, s_bad + cur, wave, ln, tid);
           __syncthreads();
         }
       }
@@ -842,6 +943,7 @@ __global__ __launch_bounds__(NW * 64, 2) void decode_rows_kernel(const DecodePar
 
     // ---- merge the token groups; write the tile, or this piece's partial -------------------------------------
     __syncthreads();  // the chunk buffers become the merge buffers
+    if (tid < NBUF) s_bad[tid] = 0;
     st.l = sum_xor<32>(st.l);
     float* mrg = (float*)smem;
     if (wn > 0) {

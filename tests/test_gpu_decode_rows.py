@@ -143,3 +143,70 @@ def test_rows_int8_scales_over_the_float32_range():
         got, want = run_case(d, out_dtype=torch.float32)
         err = np.abs(got.cpu().numpy() - want).max()
         assert err <= 2.0**-14 * np.abs(want).max(), f"2^{lo} .. 2^{hi}: {err:.3e}"
+
+
+def plant_nonfinite(c, nq, with_stale=True):
+    """Values (BF16), NaN codes (FP8) or value scales (per token) that are not finite, at a token that every query sees, at
+    several of the new ones and at each sequence's last. Returns the oracle's pools, those at zero, and the planted values
+    as [(sequence, token, head, 128 values)]. with_stale: every slot that holds no token becomes NaN too."""
+    fmt, per_token = c["fmt"], c["vs"] is not None and c["vs"].dim() == 3
+    k, v, lens, page = c["k"], c["v"].clone(), c["lens"].tolist(), c["k"].shape[1]
+    ks, vs = (None if x is None else x.clone() for x in (c["ks"], c["vs"]))
+    raw = v if fmt != "fp8" else v.view(torch.uint8)
+    slot = lambda b, t: (int(c["table"][b, t // page]), t % page)  # noqa: E731
+    if with_stale:
+        used = torch.zeros(v.shape[:2], dtype=torch.bool, device=DEV)
+        for b, n in enumerate(lens):
+            at = torch.arange(n, device=DEV)
+            used[c["table"][b, at // page].long(), at % page] = True
+        if fmt != "int8":
+            raw[~used] = float("nan") if fmt == "bf16" else 0x7F
+            k = k.clone()
+            (k if fmt == "bf16" else k.view(torch.uint8))[~used] = float("nan") if fmt == "bf16" else 0xFF
+        if per_token:
+            ks[~used], vs[~used] = float("nan"), float("nan")
+    clean_v, clean_vs, planted = v.clone(), None if vs is None else vs.clone(), []
+    heads = v.shape[2]
+    for b, n in enumerate(lens):
+        for i, t in enumerate(sorted({0 if b % 2 else n // 3, n - nq + 3, n - nq // 2, n - 2, n - 1})):
+            if not 0 <= t < n:
+                continue
+            h, ch, (e, o) = (b + i) % heads, 31 * (b + i) % 128, slot(b, t)
+            bad = torch.zeros(128)
+            if per_token:
+                x = [float("inf"), float("nan"), float("-inf")][i % 3]
+                bad = (v[e, o, h].float() * x).cpu()
+                vs[e, o, h], clean_vs[e, o, h] = x, 0.0
+            else:
+                for j, x in enumerate([float("inf"), float("-inf"), float("nan")] if fmt == "bf16" else [float("nan")] * 3):
+                    bad[(ch + j) % 128] = x
+                    raw[e, o, h, (ch + j) % 128] = x if fmt == "bf16" else 0x7F + 0x80 * (j & 1)
+                    clean_v.view(raw.dtype)[e, o, h, (ch + j) % 128] = 0
+            planted.append((b, t, h, bad.numpy()))
+    return dict(c, k=k, v=v, ks=ks, vs=vs), dict(c, k=k, v=clean_v, ks=ks, vs=clean_vs), planted
+
+
+@pytest.mark.parametrize("fmt,scales", [("bf16", None), ("fp8", "head"), ("fp8", "token"), ("int8", "token")])
+@pytest.mark.parametrize("nq,hq,hkv,lengths", [
+    (17, 4, 4, [517, 17, 129, 300]), (32, 4, 2, [517, 40, 128, 2000]), (150, 2, 2, [517, 150, 385, 256]),
+    (64, 24, 8, [3000, 65, 700]), (257, 32, 8, [2900, 257, 400, 700])])
+@pytest.mark.parametrize("page", [16, 4])
+def test_rows_values_that_are_not_finite_reach_only_the_rows_that_see_them(fmt, scales, nq, hq, hkv, lengths, page):
+    """A row gets the infinities and NaN of the tokens it sees, in their channels, and nothing of the others: of later
+    queries' tokens, and of stale slots behind a sequence's end. (Weights here are far from underflow.)"""
+    from bpt_amd import paged_decode_attention
+
+    c = make_case(fmt, lengths, hq=hq, hkv=hkv, nq=nq, page=page, scales=scales, seed=nq, outliers=False)
+    dirty, clean, planted = plant_nonfinite(c, nq)
+    scale = 0.02
+    _, want = run_case(clean, scale=scale, out_dtype=torch.float32)
+    got = paged_decode_attention(dirty["q"], dirty["k"], dirty["v"], dirty["table"], dirty["lens"], dirty["ks"], dirty["vs"],
+                                 scale=scale, max_context=max(lengths), out_dtype=torch.float32).cpu().numpy()
+    with np.errstate(invalid="ignore"):
+        for b, t, h, bad in planted:
+            first = max(t - (lengths[b] - nq), 0)  # the first query that sees token t
+            want[b, first:, h * (hq // hkv):(h + 1) * (hq // hkv)] += np.where(np.isfinite(bad), 0, bad)
+    fin = np.isfinite(want)
+    assert np.array_equal(np.isfinite(got), fin)
+    assert np.array_equal(got[~fin], want[~fin], equal_nan=True)
+    assert np.abs(got[fin] - want[fin]).max() <= 2.0**-14 * np.abs(want[fin]).max()
