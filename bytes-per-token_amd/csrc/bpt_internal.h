@@ -283,6 +283,12 @@ struct KiviParams {
 
 // The most tail tokens a KIVI call takes (a tail is shorter than a key group).
 constexpr int kKiviMaxTail = 64;
+// The waves of a workgroup take the tail's tokens four at a time in turn (16 lanes to a token): the token of a lane in
+// each round, and the rounds that cover the longest tail.
+constexpr int kivi_tail_rounds(int waves) { return (kKiviMaxTail + 4 * waves - 1) / (4 * waves); }
+constexpr __host__ __device__ int kivi_tail_token(int waves, int round, int wave, int lane) {
+  return 4 * (waves * round + wave) + (lane >> 4);
+}
 
 // Launch-ready form of bpt_kivi_quant_args: KIVI quantize-on-write of keys and values [B, Hkv, T, D].
 struct KiviQuantParams {

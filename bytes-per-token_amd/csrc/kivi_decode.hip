@@ -635,21 +635,21 @@ __device__ __forceinline__ int64_t lse_index(const KiviParams& p, int b, int hq,
   return (int64_t)b * p.l_sb + (int64_t)hq * p.l_sh + (int64_t)j * p.l_ss;
 }
 
-// This wave's share of the full-precision tail for the G query heads of (b, h): tokens 16 i + 4 wave + lane / 16,
-// folded in float32 into a wave state (base 2, reference point m, bias kBias) in LDS: s_m[r] = m_r, its largest
-// score (-inf without tokens), s_l[r] = sum_t 2^(s_rt - m_r + kBias), s_o[r][ch] = sum_t 2^(s_rt - m_r + kBias)
-// v_t[ch], where s_rt = sm_scale log2(e) q_r . k_t (fastserve integration/kv_cache.py:179-182: partial_attention
-// over the tail). s_o holds the q rows on entry (unscaled, stored by this wave).
+// This wave's share of the full-precision tail for the G query heads of (b, h): its kivi_tail_token tokens, folded in
+// float32 into a wave state (base 2, reference point m, bias kBias) in LDS: s_m[r] = m_r, its largest score (-inf
+// without tokens), s_l[r] = sum_t 2^(s_rt - m_r + kBias), s_o[r][ch] = sum_t 2^(s_rt - m_r + kBias) v_t[ch], where
+// s_rt = sm_scale log2(e) q_r . k_t (fastserve integration/kv_cache.py:179-182: partial_attention over the tail). s_o
+// holds the q rows on entry (unscaled, stored by this wave).
 //
 // What bounds it is latency, so every key and value of the wave is requested at once (16 lanes of 8 channels to
 // a token, one 16-byte load each for aligned 16-bit tails) and the call comes before the piece's chunk loop,
 // whose first chunks are in flight meanwhile. (One thread per score and per output channel, after the loop: 16
 // serial rounds of strided loads. 16 sequences, 8 KV heads, 2 rows, 2048 4-bit tokens and 17 in the tail: 54.0 us,
 // now 23.4, and 18.2 without a tail; 8-bit codes with 31 in the tail 25.7, without 20.9.)
-template <int RP>
+template <int NW, int RP>
 __device__ __forceinline__ void tail_state(const KiviParams& p, int b, int h, int wave, int lane, float* s_m, float* s_l,
                                            float (*s_o)[kHeadDim + 1]) {
-  constexpr int NI = kKiviMaxTail / 16;
+  constexpr int NI = kivi_tail_rounds(NW);
   const int T = p.tail_len;
   const int part = lane & 15;
   const int64_t at = (int64_t)b * p.tk_sb + (int64_t)h * p.tk_sh + 8 * part;
@@ -660,7 +660,7 @@ __device__ __forceinline__ void tail_state(const KiviParams& p, int b, int h, in
     u32x4 kw[NI], vw[NI];
 #pragma unroll
     for (int i = 0; i < NI; ++i) {
-      const int t = 16 * i + 4 * wave + (lane >> 4);
+      const int t = kivi_tail_token(NW, i, wave, lane);
       kw[i] = u32x4{0u, 0u, 0u, 0u};
       vw[i] = u32x4{0u, 0u, 0u, 0u};
       if (t < T) {
@@ -686,7 +686,7 @@ __device__ __forceinline__ void tail_state(const KiviParams& p, int b, int h, in
   } else {
 #pragma unroll
     for (int i = 0; i < NI; ++i) {
-      const int t = 16 * i + 4 * wave + (lane >> 4);
+      const int t = kivi_tail_token(NW, i, wave, lane);
 #pragma unroll
       for (int j = 0; j < 8; ++j) kf[i][j] = vf[i][j] = 0.0f;
       if (t < T) {
@@ -713,7 +713,7 @@ __device__ __forceinline__ void tail_state(const KiviParams& p, int b, int h, in
         a1 = fmaf(q[j + 1], kf[i][j + 1], a1);
       }
       const float x = group_sum<16>(a0 + a1) * p.qscale;
-      s[i] = 16 * i + 4 * wave + (lane >> 4) < T ? x : kNegInf;
+      s[i] = kivi_tail_token(NW, i, wave, lane) < T ? x : kNegInf;
       m = fmaxf(m, s[i]);
     }
     m = max_xor<32>(max_xor<16>(m));
@@ -756,7 +756,7 @@ __device__ __forceinline__ void zero_empty_splits(const KiviParams& p, const int
         s_o[wave][i / D][i % D] = load_float(p.q, qo + i % D, p.q_dtype);
       }
       wave_sync();
-      tail_state<RP>(p, b, h, wave, lane, s_m[wave], s_l[wave], s_o[wave]);
+      tail_state<NW, RP>(p, b, h, wave, lane, s_m[wave], s_l[wave], s_o[wave]);
       __syncthreads();
       for (int i = threadIdx.x; i < p.G * D; i += NT) {
         const int r = i / D, ch = i - r * D;
@@ -965,7 +965,7 @@ __global__ __launch_bounds__(kDecodeWaves * 64, 2) void kivi_decode_kernel(const
 #pragma unroll
       for (int c1 = 0; c1 < CPL; ++c1) s_o[wave][lane / LPR][(lane % LPR) * CPL + c1] = qf[c1];
       wave_sync();
-      tail_state<RP>(p, b, h, wave, lane, s_m[wave], s_l[wave], s_o[wave]);
+      tail_state<NW, RP>(p, b, h, wave, lane, s_m[wave], s_l[wave], s_o[wave]);
       wave_sync();
     }
 
