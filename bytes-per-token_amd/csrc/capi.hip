@@ -356,9 +356,9 @@ void line_fields(const Plan& pl, bpt::DecodeParams* p) {
 // Checks a decode call's arguments and buffers on the host and fills its launch parameters (*p, *pl); nothing
 // is launched. *empty: a batch of zero (nothing to launch).
 int decode_setup(const bpt_decode_args* a, const char* fn, const Buffers* own, bpt::DecodeParams* out, Plan* plan,
-                 bool* empty) {
+                 bool* empty, bool tiles_ok = true) {
   Plan& pl = *plan;
-  int rc = make_plan(a, &pl, true, own == nullptr);
+  int rc = make_plan(a, &pl, tiles_ok, own == nullptr);
   if (rc) return rc;
   const Buffers buf = own ? *own : Buffers{a->workspace, a->workspace_bytes, a->counters, a->counters_bytes};
   *empty = a->batch == 0;
@@ -437,11 +437,11 @@ int decode_setup(const bpt_decode_args* a, const char* fn, const Buffers* own, b
 }
 
 int paged_decode(const bpt_decode_args* a, void* stream, const bpt::LaunchEvents& ev, const char* fn,
-                 const Buffers* own = nullptr, const bpt::AppendParams* fuse = nullptr) {
+                 const Buffers* own = nullptr, const bpt::AppendParams* fuse = nullptr, bool tiles_ok = true) {
   Plan pl;
   bpt::DecodeParams p;
   bool empty;
-  int rc = decode_setup(a, fn, own, &p, &pl, &empty);
+  int rc = decode_setup(a, fn, own, &p, &pl, &empty, tiles_ok);
   if (rc) return rc;
   if (empty) {
     if (ev.start) {  // nothing to launch: the interval is empty
@@ -550,6 +550,13 @@ int bpt_paged_decode_noalloc(const bpt_decode_args* a, void* stream) {
   Plan pl;
   int rc = make_plan(a, &pl, true, false);
   if (rc) return rc;
+  // With more workgroups than the built-in plan launches (bpt_set_tuning), the tiles' partials can outgrow the array:
+  // the call then takes the vector kernel's four-row partials, if those fit.
+  const bool tiles_ok = !pl.tiles || pl.workspace <= kScratchWorkspace;
+  if (!tiles_ok) {
+    rc = make_plan(a, &pl, false, false);
+    if (rc) return rc;
+  }
   if (pl.workspace > kScratchWorkspace || pl.counters > kScratchCounters)
     return fail(BPT_ERR_INVALID_ARGUMENT,
                 "%s: the call needs %zu bytes of partials and %zu of counters; the device scratch holds %zu and %zu "
@@ -560,7 +567,7 @@ int bpt_paged_decode_noalloc(const bpt_decode_args* a, void* stream) {
   rc = scratch_for((hipStream_t)stream, &base, fn);
   if (rc) return rc;
   const Buffers own{base, kScratchWorkspace, base + kScratchWorkspace, kScratchCounters};
-  return paged_decode(a, stream, {}, fn, &own);
+  return paged_decode(a, stream, {}, fn, &own, nullptr, tiles_ok);
 }
 
 int bpt_paged_decode_timed(const bpt_decode_args* a, void* stream, void* start_event, void* stop_event) {

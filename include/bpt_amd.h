@@ -372,8 +372,10 @@ int bpt_paged_decode(const bpt_decode_args* args, void* stream);
  * resident array of the library (34 MiB of partials and 2 MiB of counters on each GPU it runs on, held until the
  * process ends), so the call allocates nothing: for callers that cannot allocate (code under HIP graph
  * capture, tight serving loops, harnesses that forbid hipMalloc). No counterpart in the reference. The
- * workspace and counters fields of args are ignored; a call whose bpt_decode_plan sizes exceed the array's
- * returns BPT_ERR_INVALID_ARGUMENT. Calls on one GPU share the array: calls that may overlap (different
+ * workspace and counters fields of args are ignored. The call has a plan of its own: that of bpt_decode_plan, but with
+ * tiles of at most 128 rows where that one takes 256 (more than 16 query rows per KV head), whose results may differ
+ * from bpt_paged_decode's in the last bits. With the built-in tuning such a call always fits the array (up to 128
+ * KV heads); any other call fits it if its bpt_decode_plan sizes do, and returns BPT_ERR_INVALID_ARGUMENT if not. Calls on one GPU share the array: calls that may overlap (different
  * streams) race and must not be issued. */
 int bpt_paged_decode_noalloc(const bpt_decode_args* args, void* stream);
 

@@ -1,6 +1,7 @@
 """GPU: bpt_paged_decode_noalloc (partials and counters in the library's device-resident array) gives exactly
 what bpt_paged_decode with a caller workspace gives, on two calls in a row (the second smaller), through the C
-ABI; a call too large for the array is refused before anything is launched."""
+ABI; a call too large for the array is refused before anything is launched. Calls that bpt_paged_decode runs in
+256-row tiles run in 128-row ones here: those are checked against the oracle."""
 
 import ctypes
 
@@ -75,3 +76,45 @@ def test_noalloc_refuses_a_call_larger_than_its_array():
     out = noalloc(make_case("fp8", [64, 65]))  # and the next call works
     torch.cuda.synchronize()
     assert torch.isfinite(out.float()).all()
+
+
+@pytest.mark.parametrize("fmt,scales", [("fp8", "head"), ("int8", "token"), ("bf16", None)])
+@pytest.mark.parametrize("nq,lengths", [
+    (16, [4096, 1000, 33, 16, 2500, 0, 700]),  # 32-row tiles, combined in the launch
+    (16, [3000]),  # and by a second launch (24 pieces of 16 KiB a tile)
+    (32, [4096, 1000, 33, 32, 2500, 0, 700]),  # 64-row tiles
+    (32, [3000]),
+    (64, [300, 64, 129, 256, 0, 70, 65]),  # 128-row tiles
+    (64, [4096, 1000, 64, 2500])])
+def test_noalloc_takes_many_rows(fmt, scales, nq, lengths):
+    small = make_case(fmt, [200, 17], scales=scales, nq=1, seed=6)
+    for c in (make_case(fmt, lengths, scales=scales, nq=nq, seed=nq), small):
+        got = noalloc(c)
+        want = reference(c)
+        torch.cuda.synchronize()
+        assert torch.equal(got, want), f"{fmt} Q={c['q'].shape[1]}: differs from bpt_paged_decode"
+
+
+@pytest.mark.parametrize("fmt,scales", [("fp8", "head"), ("int8", "token"), ("bf16", None)])
+def test_noalloc_takes_128_row_tiles_where_the_plan_takes_256(fmt, scales):
+    from bpt_amd import decode_plan
+
+    c = make_case(fmt, [4096, 1000, 256, 2500, 0, 700, 3333], scales=scales, nq=256, seed=9)
+    ws = decode_plan(c["q"], c["k"], c["v"], c["table"], c["lens"], c["ks"], c["vs"], scale=0.1, max_context=4096)[2]
+    assert ws > 34 << 20  # more than the array holds
+    got = noalloc(c)
+    check(got, run_case(c)[1], f"{fmt} 256 queries against the oracle")
+    small = make_case(fmt, [200, 17], scales=scales, seed=6)
+    assert torch.equal(noalloc(small), reference(small))
+
+
+def test_noalloc_takes_the_vector_kernel_where_tuned_tiles_outgrow_the_array():
+    c = make_case("fp8", [4096, 1000, 64, 2500], nq=64, seed=10)
+    want = run_case(c)[1]
+    _lib.set_tuning(groups_per_cu=4)
+    try:
+        got = noalloc(c)
+        torch.cuda.synchronize()
+    finally:
+        _lib.set_tuning()
+    check(got, want, "four workgroups per CU")
