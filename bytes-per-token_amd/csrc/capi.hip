@@ -1004,8 +1004,13 @@ int bpt_page_read_probe(const bpt_decode_args* a, float* partial_sums, int64_t* 
                         void* start_event, void* stop_event) {
   const char* fn = "bpt_page_read_probe";
   Plan pl;
-  int rc = make_plan(a, &pl, false);  // the probe reads in the other kernels' order
+  int rc = make_plan(a, &pl);
   if (rc) return rc;
+  // A many-row tile reads a chunk once for all of its rows, as a segment of the other kernels does: the walk goes through
+  // it kMfmaChunk tokens at a time, over the whole sequence.
+  if (pl.tiles) pl.chunk = bpt::kMfmaChunk;
+  if ((int64_t)a->batch * ((pl.len_cap + pl.chunk - 1) / pl.chunk) > 0x7fffffffLL / pl.HR)
+    return fail(BPT_ERR_INVALID_ARGUMENT, "%s: batch x context x heads too large", fn);
   const int64_t g = a->batch > 0 ? pl.grid : 0;  // the decode's workgroups
   if (num_groups) *num_groups = g;
   if (!partial_sums) return BPT_OK;

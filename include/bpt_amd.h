@@ -450,7 +450,9 @@ int bpt_read_probe_timed(const void* buf, uint64_t bytes, float* partial_sums, v
 /* The page-read probe: every K and V row (and per-token scale) that bpt_paged_decode over the same args
  * reads, fetched through the same block table and context lengths, in the decode's own order (its segments,
  * workgroup ranges and chunks, the same number of workgroups) with no attention math and no merges (one float
- * per workgroup into partial_sums). It is the read floor of a decode call's own access pattern. Call with
+ * per workgroup into partial_sums). It is the read floor of a decode call's own access pattern. A call of the many-row
+ * kernel is read once per tile of its rows, over the same workgroups, in 32-token steps and over whole sequences (also
+ * the tokens that only later queries see). Call with
  * partial_sums = NULL to get the workgroup count in *num_groups. Optional events as bpt_read_probe_timed
  * (both or neither). Uses the shape, cache, scale, table and length fields of args. No reference
  * counterpart. */

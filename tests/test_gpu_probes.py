@@ -68,7 +68,8 @@ def page_checksums(w, groups):
     from bpt_amd.paged_attention import _plan
 
     a, _, _ = _plan(*w.args(), **{k: v for k, v in w.kwargs().items()})
-    chunk, rows = a.chunk_tokens, a.num_queries * (a.num_q_heads // a.num_kv_heads)
+    chunk = a.chunk_tokens if a.rows_per_group <= 16 else 32  # many-row tiles are walked 32 tokens at a time
+    rows = a.num_queries * (a.num_q_heads // a.num_kv_heads)
     n_rg = -(-rows // a.rows_per_group)
     k = w.k_cache.contiguous().view(torch.uint8).cpu().numpy()
     v = w.v_cache.contiguous().view(torch.uint8).cpu().numpy()
@@ -115,6 +116,21 @@ def test_page_read_probe_reads_the_calls_pages(name):
     want = page_checksums(w, got.size)
     assert got.shape == want.shape
     assert np.array_equal(got, want)
+
+
+@pytest.mark.parametrize("fmt,scales,queries", [("fp8", "head", 9), ("int8", "token", 40), ("bf16", "none", 150), ("fp8", "head", 1024)])
+def test_page_read_probe_reads_many_row_tiles_once(fmt, scales, queries):
+    from bpt_amd import measure, workloads
+    from bpt_amd.paged_attention import _plan
+
+    w = workloads.make(shape=workloads.Shape("t", 3, 16, 8, fmt, scales, (queries, queries + 1500), queries=queries), device="cuda", seed=queries)
+    plan, _, _ = _plan(*w.args(), **w.kwargs())
+    assert plan.rows_per_group == {9: 32, 40: 128, 150: 128, 1024: 256}[queries]
+    probe = measure.PageReadProbe(*w.args(), **w.kwargs())
+    assert probe.partial.numel() == plan.grid_groups  # the decode's workgroups
+    probe.run()
+    torch.cuda.synchronize()
+    assert np.array_equal(probe.partial.cpu().numpy(), page_checksums(w, plan.grid_groups))
 
 
 def test_page_read_probe_query_and_events():
