@@ -80,6 +80,8 @@ struct RowsCfg {
   static constexpr int kOut = BM * (kHeadDim + 4) * 4 + BM * 4;
   static constexpr int kSmem = NBUF * kBuf > kMerge ? (NBUF * kBuf > kOut ? NBUF * kBuf : kOut)
                                                     : (kMerge > kOut ? kMerge : kOut);
+  // Whether pieces can be combined in the launch: two of the largest tiles' already call for a second one (rows_two_pass).
+  static constexpr bool kInLaunch = 2 * BM * kHeadDim * 4 < kRowsTwoPassBytes;
   static_assert(NW % WM == 0 && TW % 32 == 0 && (CT / 16) % NW == 0, "tile shape");
 };
 
@@ -1019,7 +1021,7 @@ __global__ __launch_bounds__(NW * 64, 2) void decode_rows_kernel(const DecodePar
         const int row = t * BM + r;
         const int qi = row / p.G;
         rows_write4(p, b, qi, h * p.G + (row - qi * p.G), ch, o, s_lse[r], packed);
-      } else if (p.two_pass) {
+      } else if (!C::kInLaunch || p.two_pass) {
         *(f32x4*)(p.ws_out + (slot * BM + r) * D + ch) = o;
         if (ch == 0) p.ws_lse[slot * BM + r] = s_lse[r];
       } else {
@@ -1028,16 +1030,18 @@ __global__ __launch_bounds__(NW * 64, 2) void decode_rows_kernel(const DecodePar
         if (ch == 0) ws_store(p.ws_lse + slot * BM + r, s_lse[r]);
       }
     }
-    if (!whole && !p.two_pass) {
-      const int seg = (b * Hkv + h) * T + t;
-      const int n = (int)(g_last - g_first + 1);
-      ws_publish();
-      __syncthreads();
-      if (tid == 0) s_last = ws_arrive(p.counters + seg) == (unsigned)n - 1u;
-      __syncthreads();
-      if (s_last) {
-        rows_combine<BM, NT>(p, b, h, t, g_first, n, live, packed, tid);
-        if (tid == 0) __hip_atomic_store(p.counters + seg, 0u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    if constexpr (C::kInLaunch) {
+      if (!whole && !p.two_pass) {
+        const int seg = (b * Hkv + h) * T + t;
+        const int n = (int)(g_last - g_first + 1);
+        ws_publish();
+        __syncthreads();
+        if (tid == 0) s_last = ws_arrive(p.counters + seg) == (unsigned)n - 1u;
+        __syncthreads();
+        if (s_last) {
+          rows_combine<BM, NT>(p, b, h, t, g_first, n, live, packed, tid);
+          if (tid == 0) __hip_atomic_store(p.counters + seg, 0u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+        }
       }
     }
     if (!more) break;

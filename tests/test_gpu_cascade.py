@@ -85,6 +85,20 @@ def test_prefix_pass_as_one_sequence(fmt, scales, batch, q_heads, queries, pages
     close(got, want, f"{fmt} {batch} x {queries}, {pages} pages")
 
 
+@pytest.mark.parametrize("fmt,scales,queries,q_heads", [("fp8", "head", 20, 16), ("bf16", "none", 9, 16), ("int8", "token", 300, 16)])
+def test_long_suffixes_of_many_rows_merge_in_the_second_launch(fmt, scales, queries, q_heads):
+    """40, 18 and 600 rows per KV head over thousands of own tokens: the suffix pass's pieces are combined by a second
+    launch, which merges the prefix's partial into float32 and bf16 results."""
+    from bpt_amd import cascade_decode_attention, workloads
+
+    shape = workloads.Shape("t", 2, q_heads, 8, fmt, scales, (3300, 4300), queries=queries, shared_prefix_pages=9)
+    w = workloads.make(shape=shape, device="cuda", seed=queries)
+    want, _ = oracle_of(w)
+    for dtype in (torch.float32, torch.bfloat16):
+        got = cascade_decode_attention(*w.args(), **w.kwargs(), prefix_pages=9, out_dtype=dtype, context_lens_host=w.lengths)
+        close(got, want, f"{fmt} {queries} queries {dtype}")
+
+
 def test_empty_suffixes_give_the_prefix_alone():
     from bpt_amd import cascade_decode_attention, workloads
 

@@ -74,6 +74,25 @@ def test_rows_two_launches_replay_in_a_graph(nq):
         torch.cuda.synchronize()
 
 
+def test_rows_two_launches_timed():
+    """The timed entry point over a call of two launches: the start event on the first, the stop event on the second."""
+    from bpt_amd import paged_decode_attention
+
+    c = make_case("fp8", [3000, 450], hq=16, hkv=2, nq=100, seed=100)
+    args = (c["q"], c["k"], c["v"], c["table"], c["lens"], c["ks"], c["vs"])
+    want = paged_decode_attention(*args, scale=0.09, max_context=3000)
+    start, mid, stop, end = (torch.cuda.Event(enable_timing=True) for _ in range(4))
+    for e in (start, mid, stop, end):
+        e.record()
+    torch.cuda.synchronize()
+    start.record()
+    got = paged_decode_attention(*args, scale=0.09, max_context=3000, _events=(mid.cuda_event, stop.cuda_event))
+    end.record()
+    torch.cuda.synchronize()
+    assert torch.equal(got, want)
+    assert 0 < mid.elapsed_time(stop) <= start.elapsed_time(end)
+
+
 @pytest.mark.parametrize("num_splits", [1, 3, 1000])
 @pytest.mark.parametrize("nq", [10, 20, 40])
 def test_rows_forced_splits(num_splits, nq):
