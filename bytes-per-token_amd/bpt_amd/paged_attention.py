@@ -166,8 +166,11 @@ def decode_kernel_name(
 
 
 # Per (device, stream): one partials workspace and one zero-filled counter buffer. The kernel leaves the
-# counters at zero, so calls issued in order on one stream share them; other streams get their own.
+# counters at zero, so calls issued in order on one stream share them; other streams get their own. A buffer that
+# a larger call outgrows is kept: a graph captured on the stream goes on using it at every replay. Each is at least
+# twice the one before, so those kept are smaller together than the one in use.
 _BUFFERS: dict[tuple[str, int, int], torch.Tensor] = {}
+_OUTGROWN: list[torch.Tensor] = []
 _GRAIN = 1 << 20
 
 
@@ -178,6 +181,9 @@ def cached_buffer(kind: str, device: torch.device, stream: int, nbytes: int) -> 
     buf = _BUFFERS.get(key)
     if buf is None or buf.numel() < nbytes:
         size = max((nbytes + _GRAIN - 1) // _GRAIN * _GRAIN, _GRAIN)
+        if buf is not None:
+            _OUTGROWN.append(buf)
+            size = max(size, 2 * buf.numel())
         buf = torch.zeros(size, dtype=torch.uint8, device=device)
         _BUFFERS[key] = buf
     return buf
