@@ -151,7 +151,20 @@ constexpr int kMfmaChunk = 32;
 // 4 x 300, 32 heads (480) 51 : 47.
 constexpr int kRowsChunk = 128;
 constexpr int64_t kRowsWideChunks = 8 * kComputeUnits;
-constexpr int rows_tile(int rows) { return rows <= 32 ? 32 : rows <= 64 ? 64 : 128; }
+// Rows of a tile below that: the fewest that hold a KV head's rows, or that still leave no more than one (tile, chunk) unit
+// for each CU (`segments`: sequences x KV heads, `chunks`: of the longest sequence). Larger tiles would leave most of the
+// chip idle there, and their pieces take the one CU that combines them longer. Measured, kernel times, medians over some
+// 600 calls of 80 to 256 rows for each format against 128-row tiles: up to 256 units of 32 rows FP8 -15 %, BF16 -18 %,
+// INT8 -22 % (FP8 128 rows x 300 tokens, 2 heads 23.2 -> 18.0 us; the vector kernel 20.0), up to 256 units of 64 rows -11,
+// -12 and -17 %; beyond that they lose 5 to 30 %. For 33 to 64 rows 32-row tiles take 0.98 (INT8 0.95) of the time of
+// 64-row ones, but 1.05 over one chunk; and 1.02 with an f16 q over BF16, whose q in two parts spills most there: those
+// start at 64.
+constexpr int rows_tile(int rows, int64_t segments, int64_t chunks, bool q_split) {
+  if (rows <= 32) return 32;
+  if (!q_split && (chunks > 1 || rows > 64) && segments * ((rows + 31) / 32) * chunks <= kComputeUnits) return 32;
+  if (rows <= 64 || segments * ((rows + 63) / 64) * chunks <= kComputeUnits) return 64;
+  return 128;
+}
 constexpr int rows_groups_per_cu(int tile) { return tile == 32 ? 2 : 1; }
 constexpr int kRowsMinChunks = 1;
 constexpr int kRowsPieceCost = 2;

@@ -61,14 +61,40 @@ std::mutex g_tuning_mutex;
 
 size_t align256(size_t x) { return (x + 255) & ~(size_t)255; }
 
-// Whether a call with more than 16 rows per KV head takes the many-row kernel: a bf16 or f16 q (an f32 q keeps the
-// vector kernel's float32 products), 16 token strides of a page within 32 bits, and a tile line that fits its LDS.
-bool takes_tiles(const bpt_decode_args* a, int rows, int tile) {
+// Chunks of each of the vector kernel's equal partitions over `chunks` of them (kAlignedMaxChunksBf16): a power of two
+// that gives about 4 sqrt(chunks) partitions, then as many times that as kAlignedMaxGrid workgroups need.
+int64_t aligned_partition(int64_t chunks) {
+  int64_t target = (int64_t)(4.0 * std::sqrt((double)chunks));
+  target = target < 1 ? 1 : (target > bpt::kAlignedMaxGrid ? bpt::kAlignedMaxGrid : target);
+  int64_t per = 1;
+  while (per * 2 <= chunks / target) per *= 2;
+  const int64_t parts = (chunks + per - 1) / per;
+  if (parts > bpt::kAlignedMaxGrid) per *= (parts + bpt::kAlignedMaxGrid - 1) / bpt::kAlignedMaxGrid;
+  return per;
+}
+
+// Whether a call with more than 16 rows per KV head (`len_cap` tokens at most) takes the many-row kernel: a bf16 or f16 q
+// (an f32 q keeps the vector kernel's float32 products), 16 token strides of a page within 32 bits, a tile line that fits
+// its LDS, and no BF16 cache whose rows the vector kernel's partitions cover better.
+bool takes_tiles(const bpt_decode_args* a, int rows, int tile, int64_t len_cap) {
   if (rows <= bpt::kMfmaRows || a->q_dtype == BPT_F_F32) return false;
   const int64_t stok = a->kv_stride_token * (a->kv_dtype == BPT_KV_BF16 ? 2 : 1);
   if (stok < 0 || 16 * stok >= (int64_t(1) << 31)) return false;
   const int64_t tiles = ((int64_t)rows + tile - 1) / tile;
-  return (int64_t)a->batch * (tiles + 1) <= bpt::kRowsMaxLine;
+  if ((int64_t)a->batch * (tiles + 1) > bpt::kRowsMaxLine) return false;
+  if (a->kv_dtype != BPT_KV_BF16 || a->num_splits > 0) return true;
+  // Small BF16 calls: where a sequence's chunks are whole equal partitions of at most eight, the vector kernel's piece is
+  // short (12 to 17 us in all) and nothing is merged across sequences, while a tile waits for its pieces' combine: from
+  // four partitions of a sequence on the tiles took 1.05 to 1.47 of its time (100 calls; 24 rows x 512 tokens, 8 heads
+  // 14.4 us against 17.9; with ragged lengths below the same bound 0.94 to 1.27), below that 0.83 to 1.09. An f16 q, which
+  // the tiles take in two parts, loses from two partitions on, and for one sequence always: 0.94 to 1.58. Of other such
+  // calls the vector kernel would win the few that the bound on the lengths does not tell from the rest (ragged batches
+  // of two to four sequences of 300 to 700 tokens, up to 1.29; with equal lengths 0.6 to 0.8).
+  const int64_t chunk = bpt::decode_chunk_tokens(a->kv_dtype, 4);
+  const int64_t nb = (len_cap + chunk - 1) / chunk;
+  const int64_t per = aligned_partition((int64_t)a->batch * a->num_kv_heads * ((rows + 3) / 4) * nb);
+  if (nb == 0 || per > 8 || nb % per) return true;
+  return a->q_dtype == BPT_F_F16 ? a->batch > 1 && nb == per : nb < 10 || nb < 4 * per;
 }
 
 // tiles_ok: whether the many-row kernel may be chosen; wide_ok: and its 256-row tiles (whose partials outgrow the
@@ -112,13 +138,15 @@ int make_plan(const bpt_decode_args* a, Plan* pl, bool tiles_ok = true, bool wid
   // from 5 rows on (with fewer, the vector kernel reads each page once too and its INT8 decode is cheaper).
   pl->mfma = pl->rows <= bpt::kMfmaRows && ((a->kv_dtype == BPT_KV_FP8_E4M3FN && pl->rows >= bpt::kMfmaMinRows) ||
                                             (a->kv_dtype == BPT_KV_INT8 && pl->rows >= bpt::kMfmaMinRowsInt8));
-  int tile = bpt::rows_tile(pl->rows);
-  if (wide_ok && pl->rows > tile) {
-    const int64_t reach = (int64_t)a->max_blocks_per_seq * a->page_size;
-    const int64_t chunks = ((a->max_context < reach ? a->max_context : reach) + bpt::kRowsChunk - 1) / bpt::kRowsChunk;
-    if ((int64_t)((pl->rows + 255) / 256) * a->num_kv_heads * a->batch * chunks >= bpt::kRowsWideChunks) tile = 256;
-  }
-  pl->tiles = tiles_ok && takes_tiles(a, pl->rows, tile);
+  // Whatever the tile, so that the products below fit.
+  if ((int64_t)a->num_kv_heads * ((pl->rows + 255) / 256) > (1 << 20))
+    return fail(BPT_ERR_INVALID_ARGUMENT, "%s: too many KV heads x row groups", fn);
+  const int64_t reach = (int64_t)a->max_blocks_per_seq * a->page_size;
+  const int64_t tile_chunks = ((a->max_context < reach ? a->max_context : reach) + bpt::kRowsChunk - 1) / bpt::kRowsChunk;
+  const int64_t segments = (int64_t)a->batch * a->num_kv_heads;
+  int tile = bpt::rows_tile(pl->rows, segments, tile_chunks, a->kv_dtype == BPT_KV_BF16 && a->q_dtype == BPT_F_F16);
+  if (wide_ok && pl->rows > 128 && segments * ((pl->rows + 255) / 256) * tile_chunks >= bpt::kRowsWideChunks) tile = 256;
+  pl->tiles = tiles_ok && takes_tiles(a, pl->rows, tile, a->max_context < reach ? a->max_context : reach);
   pl->rows_per_group = pl->tiles ? tile : pl->mfma ? bpt::kMfmaRows : (pl->rows <= 1 ? 1 : (pl->rows <= 2 ? 2 : 4));
   pl->n_rg = (pl->rows + pl->rows_per_group - 1) / pl->rows_per_group;
   const int64_t hr = (int64_t)a->num_kv_heads * pl->n_rg;
@@ -181,12 +209,7 @@ int make_plan(const bpt_decode_args* a, Plan* pl, bool tiles_ok = true, bool wid
       // chunks when every sequence has the same length (the kernel checks); the launch keeps the line
       // cut's workgroups for ragged batches, the rest of them leaving at once otherwise. One sequence
       // is never ragged: its partitions are fixed here (no piece cost, no check in the kernel).
-      int64_t target = (int64_t)(4.0 * std::sqrt((double)bound_c));
-      target = target < 1 ? 1 : (target > bpt::kAlignedMaxGrid ? bpt::kAlignedMaxGrid : target);
-      int64_t per = 1;
-      while (per * 2 <= bound_c / target) per *= 2;
-      const int64_t parts = (bound_c + per - 1) / per;
-      if (parts > bpt::kAlignedMaxGrid) per *= (parts + bpt::kAlignedMaxGrid - 1) / bpt::kAlignedMaxGrid;
+      const int64_t per = aligned_partition(bound_c);
       const int64_t equal = (bound_c + per - 1) / per;
       if (a->batch == 1) {
         pl->per_forced = per;

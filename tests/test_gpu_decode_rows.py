@@ -26,6 +26,26 @@ def test_rows_at_tile_edges(fmt, scales, nq, hq, hkv):
     assert got[1].float().abs().sum().item() == 0  # no tokens: zeros
 
 
+def longer_bound(c, context=8192):
+    """The case with block tables for `context` tokens: calls bounded by that take the tiles of a large call."""
+    page = c["k"].shape[1]
+    return dict(c, table=torch.nn.functional.pad(c["table"], (0, context // page - c["table"].shape[1])))
+
+
+@pytest.mark.parametrize("fmt,scales", FORMATS)
+@pytest.mark.parametrize("nq,hq,hkv,tile", [(16, 4, 2, 32), (11, 6, 2, 64), (32, 4, 2, 64), (13, 10, 2, 128), (64, 2, 1, 128), (43, 3, 1, 128), (150, 4, 2, 128)])
+def test_rows_at_tile_edges_under_a_longer_bound(fmt, scales, nq, hq, hkv, tile):
+    """The same edges in the tiles that large calls take: a bound on the lengths far above them (their own bound would give
+    32- or 64-row tiles)."""
+    from bpt_amd import decode_plan
+
+    c = longer_bound(make_case(fmt, [517, 0, nq, 128, 129, 1, 260], hq=hq, hkv=hkv, nq=nq, scales=scales, seed=nq))
+    plan = decode_plan(c["q"], c["k"], c["v"], c["table"], c["lens"], c["ks"], c["vs"], scale=0.1, max_context=8192)
+    assert plan[1] == 128 and plan[2] == -(-2 * plan[0] * tile * 129 * 4 // 256) * 256
+    got, want = run_case(c, max_context=8192)
+    check(got, want, f"{fmt}/{scales} {nq} queries, {hq}/{hkv} heads")
+
+
 @pytest.mark.parametrize("fmt,scales", FORMATS)
 @pytest.mark.parametrize("page", [1, 2, 8, 16, 128])
 @pytest.mark.parametrize("q_dtype", [torch.bfloat16, torch.float16])
@@ -131,8 +151,9 @@ def test_rows_negative_scale_and_lse_and_repeats():
 
 
 @pytest.mark.parametrize("q_dtype", [torch.bfloat16, torch.float16])
+@pytest.mark.parametrize("context", [64, 8192])  # the second takes tiles of up to 256 rows
 @pytest.mark.parametrize("hq,nq", [(17, 1), (33, 1), (65, 1), (300, 1), (64, 40)])
-def test_rows_int8_weights_keep_all_24_bits(hq, nq, q_dtype):
+def test_rows_int8_weights_keep_all_24_bits(hq, nq, q_dtype, context):
     """One visible token with zero keys: its weight is 2^4 times its float32 value scale, so a code that is a power of two
     gives that scale times the code exactly, if the weight keeps its 24 bits and its exponent (2^-60 .. 2^90)."""
     from bpt_amd import paged_decode_attention
@@ -144,10 +165,11 @@ def test_rows_int8_weights_keep_all_24_bits(hq, nq, q_dtype):
     v = codes[torch.randint(5, k.shape, generator=g, device=DEV)]
     vs = (torch.rand(k.shape[:3], generator=g, device=DEV) + 1) * torch.exp2(torch.randint(-60, 91, k.shape[:3], generator=g, device=DEV).float())
     ks = torch.ones_like(vs)
-    table = torch.arange(b * 4, dtype=torch.int32, device=DEV).view(b, 4)
+    table = torch.zeros((b, context // 16), dtype=torch.int32, device=DEV)
+    table[:, :4] = torch.arange(b * 4, dtype=torch.int32, device=DEV).view(b, 4)
     lens = torch.full((b,), t, dtype=torch.int32, device=DEV)
     q = torch.randn((b, nq, hq, 128), generator=g, device=DEV).to(q_dtype)
-    got = paged_decode_attention(q, k, v, table, lens, ks, vs, scale=0.1, max_context=t, out_dtype=torch.float32)
+    got = paged_decode_attention(q, k, v, table, lens, ks, vs, scale=0.1, max_context=context, out_dtype=torch.float32)
     want = v.view(b, 64, 128)[:, 0].float() * vs.view(b, 64)[:, :1]
     assert torch.equal(got[:, 0], want[:, None].expand(b, hq, 128))  # the first query sees the first token alone
 
@@ -210,17 +232,19 @@ def plant_nonfinite(c, nq, with_stale=True):
     (17, 4, 4, [517, 17, 129, 300]), (32, 4, 2, [517, 40, 128, 2000]), (150, 2, 2, [517, 150, 385, 256]),
     (64, 24, 8, [3000, 65, 700]), (257, 32, 8, [2900, 257, 400, 700])])
 @pytest.mark.parametrize("page", [16, 4])
-def test_rows_values_that_are_not_finite_reach_only_the_rows_that_see_them(fmt, scales, nq, hq, hkv, lengths, page):
+@pytest.mark.parametrize("bound", [None, 8192])
+def test_rows_values_that_are_not_finite_reach_only_the_rows_that_see_them(fmt, scales, nq, hq, hkv, lengths, page, bound):
     """A row gets the infinities and NaN of the tokens it sees, in their channels, and nothing of the others: of later
     queries' tokens, and of stale slots behind a sequence's end. (Weights here are far from underflow.)"""
     from bpt_amd import paged_decode_attention
 
     c = make_case(fmt, lengths, hq=hq, hkv=hkv, nq=nq, page=page, scales=scales, seed=nq, outliers=False)
+    c = c if bound is None else longer_bound(c, bound)
     dirty, clean, planted = plant_nonfinite(c, nq)
     scale = 0.02
     _, want = run_case(clean, scale=scale, out_dtype=torch.float32)
     got = paged_decode_attention(dirty["q"], dirty["k"], dirty["v"], dirty["table"], dirty["lens"], dirty["ks"], dirty["vs"],
-                                 scale=scale, max_context=max(lengths), out_dtype=torch.float32).cpu().numpy()
+                                 scale=scale, max_context=bound or max(lengths), out_dtype=torch.float32).cpu().numpy()
     with np.errstate(invalid="ignore"):
         for b, t, h, bad in planted:
             first = max(t - (lengths[b] - nq), 0)  # the first query that sees token t
