@@ -36,9 +36,9 @@
 // A token that a row does not see must add nothing to it, and the split weights must not turn an infinity into NaN, but
 // the MFMAs multiply every value by every weight and by every part of it, zeros included. So values that are not finite
 // (and per-token value scales that are not) are replaced by zeros on their way into LDS, and the rows that see them get
-// them added one by one (rows_add_nonfinite), which finite data never pays for; the look at the values costs BF16 caches
-// 1 to 2 % (2048 + 2048 tokens, 16 heads 132.5 -> 134.2 us, 512 + 8192, 32 heads 170 -> 171, with an f16 q 187 -> 192) and
-// the others nothing that shows (FP8 111 -> 110).
+// them added one by one (rows_add_nonfinite), which finite data never pays for; the look at the values, one dot product
+// with zero per two of them, costs BF16 caches 1 to 3 % (2048 + 2048 tokens, 16 heads 134 -> 137 us, 512 + 8192, 32 heads
+// 169 -> 171, with an f16 q 191 -> 196) and the others nothing that shows (FP8 111 -> 110).
 #pragma once
 
 #include <type_traits>
@@ -53,7 +53,6 @@ typedef float f32x4 __attribute__((ext_vector_type(4)));
 typedef float f32x16 __attribute__((ext_vector_type(16)));
 typedef uint32_t u32x2 __attribute__((ext_vector_type(2)));
 typedef uint32_t u32x4 __attribute__((ext_vector_type(4)));
-typedef uint16_t u16x2 __attribute__((ext_vector_type(2)));
 
 template <int KV_, int SK_, bool PU_, bool QF16_, int WM_, int NW_, int NBUF_>
 struct RowsCfg {
@@ -275,11 +274,12 @@ __device__ __forceinline__ void rows_store(const DecodeParams& p, const RowsStag
                           {s.v[u][1].x, s.v[u][1].y, s.v[u][1].z, s.v[u][1].w},
                           {s.v[u][2].x, s.v[u][2].y, s.v[u][2].z, s.v[u][2].w},
                           {s.v[u][3].x, s.v[u][3].y, s.v[u][3].z, s.v[u][3].w}};
-      u16x2 top = {0, 0};
+      const bf16x2 zero = {(__bf16)0.0f, (__bf16)0.0f};
+      float nan = 0.0f;  // what 0 times an infinity or NaN leaves
 #pragma unroll
       for (int i = 0; i < 16; ++i)
-        top = __builtin_elementwise_max(top, __builtin_bit_cast(u16x2, w[i >> 2][i & 3] & 0x7fff7fffu));
-      if (__any(top.x >= 0x7f80 || top.y >= 0x7f80)) {
+        nan = __builtin_amdgcn_fdot2_f32_bf16(__builtin_bit_cast(bf16x2, w[i >> 2][i & 3]), zero, nan, false);
+      if (__any(nan != 0.0f)) {
         *bad = kk + 1;
 #pragma unroll
         for (int i = 0; i < 16; ++i) {
