@@ -3,7 +3,7 @@
 When sequences start with the same pages (a system prompt, or the branches of a speculative verify step;
 fastserve's prefix cache decides the sharing, kv/prefix_cache.py:42-140), plain paged decode reads the
 shared pages once per sequence. The cascade reads them once per 16 query rows of the whole group, or once per
-128 or 256 of them where the group's rows and the prefix are many (_one_sequence):
+tile of up to 256 of them where the group's rows and the prefix are many (_one_sequence):
 
 1. Prefix pass. All queries of a group (members x Q queries x G heads per KV head) attend the group's
    `prefix_pages` shared pages, a group of rows at a time, non-causally (every query sits after the prefix), and
@@ -12,8 +12,8 @@ shared pages once per sequence. The cascade reads them once per 16 query rows of
    result is merged with its prefix partial as kernels/reference.py:205-211 merges split partials, so the
    output is the attention over the whole context.
 
-Both passes are the library's paged decode kernels (two launches in all, plus one per extra group); the
-merge happens in the suffix pass's final write. The result equals `paged_decode_attention` on the same
+Both passes are calls of the library's paged decode (one per group and one for the suffixes; a call is one launch, or two
+where a large call's split tiles are combined by a second one); the merge happens in the suffix pass's final write. The result equals `paged_decode_attention` on the same
 inputs up to float32 rounding.
 
 Requirements: every sequence of a group holds the group's prefix in its first `prefix_pages` block-table
@@ -40,16 +40,18 @@ def _rows_per_pass(total_queries: int, heads_per_kv: int) -> int:
     return best
 
 
-def _one_sequence(rows: int, prefix: int, q_dtype: torch.dtype, kv_dtype: torch.dtype) -> bool:
+def _one_sequence(rows: int, prefix: int, kv_heads: int, q_dtype: torch.dtype, kv_dtype: torch.dtype) -> bool:
     """Whether the prefix pass takes all of a group's rows (queries times query heads per KV head) as one sequence, on
-    the many-row kernel: more than 16 rows of a bf16 or f16 q, and rows x prefix tokens large.
+    the many-row kernel: more than 16 rows of a bf16 or f16 q, and rows x prefix tokens x KV heads large.
 
-    Measured, groups of 16 rows against one sequence, 8 KV heads (us): BF16 caches (whose groups are computed 4 rows at
-    a time) 20 rows x 512 tokens 15 : 20, 48 x 4096 54 : 24, 64 x 8192 101 : 30; FP8 64 x 8192 22 : 28, 512 x 1024
-    17 : 27, 256 x 16384 79 : 61; INT8 128 x 8192 39 : 36.
+    The product is the pass's work, and where the line lies does not depend on how it is made up. Measured, kernel times
+    of one sequence over those of groups of 16 rows (fewest .. most, at 1 to 8 KV heads, 20 to 2048 rows and 256 to 32768
+    tokens): BF16 caches, whose groups are computed 4 rows at a time, 0.91 .. 1.11 at 2^18, 0.71 .. 0.95 at 2^19, 0.42 ..
+    0.80 at 2^20; INT8 0.82 .. 1.23 at 2^23, 0.74 .. 0.93 at 2^24; FP8 0.98 .. 1.46 at 2^23, 0.83 .. 1.12 at 2^24, 0.71 ..
+    0.85 at 2^25.
     """
-    enough = 1 << 16 if kv_dtype == torch.bfloat16 else 1 << 20
-    return rows > 16 and q_dtype != torch.float32 and rows * prefix >= enough
+    enough = {torch.bfloat16: 1 << 19, torch.int8: 1 << 24}.get(kv_dtype, 3 << 23)
+    return rows > 16 and q_dtype != torch.float32 and rows * prefix * kv_heads >= enough
 
 
 def cascade_decode_attention(
@@ -110,7 +112,7 @@ def cascade_decode_attention(
     part_lse = torch.empty((b, nq, hq), dtype=torch.float32, device=dev)
     for s, e in groups:
         total = (e - s) * nq
-        whole = _one_sequence(total * heads_per_kv, prefix, q4.dtype, k_cache.dtype)
+        whole = _one_sequence(total * heads_per_kv, prefix, hkv, q4.dtype, k_cache.dtype)
         qv = total if whole else _rows_per_pass(total, heads_per_kv)
         nv = total // qv
         table = block_table[s, :prefix_pages].expand(nv, prefix_pages)

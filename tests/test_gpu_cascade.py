@@ -68,17 +68,20 @@ def test_two_groups_with_their_own_prefix_pages(fmt, scales, q_heads, queries):
 
 @pytest.mark.parametrize("fmt,scales,batch,q_heads,queries,pages", [
     ("bf16", "none", 9, 16, 2, 113), ("bf16", "none", 9, 16, 2, 114), ("bf16", "none", 7, 64, 1, 200),
-    ("fp8", "head", 32, 64, 2, 127), ("fp8", "head", 32, 64, 2, 128), ("int8", "token", 33, 64, 2, 128)])
+    ("fp8", "head", 32, 64, 2, 127), ("fp8", "head", 32, 64, 2, 128), ("int8", "token", 33, 64, 2, 128),
+    ("fp8", "head", 32, 64, 2, 383), ("fp8", "head", 32, 64, 2, 384), ("int8", "token", 33, 64, 2, 248), ("int8", "token", 33, 64, 2, 249)])
 @pytest.mark.parametrize("q_dtype", [torch.bfloat16, torch.float16])
 def test_prefix_pass_as_one_sequence(fmt, scales, batch, q_heads, queries, pages, q_dtype):
-    """Both sides of the line between 16-row groups and one sequence (36 rows x 1808 / 1824 tokens in BF16, 512 rows x
-    2032 / 2048 in FP8), and row counts that end inside a tile."""
-    from bpt_amd import cascade_decode_attention, workloads
+    """Both sides of the line between 16-row groups and one sequence, at 8 KV heads (36 rows x 1808 / 1824 tokens in BF16,
+    512 x 6128 / 6144 in FP8, 528 x 3968 / 3984 in INT8), and row counts that end inside a tile."""
+    from bpt_amd import cascade, cascade_decode_attention, workloads
 
     shape = workloads.Shape("t", batch, q_heads, 8, fmt, scales, (pages * 16 + 2, pages * 16 + 60), queries=queries,
                             shared_prefix_pages=pages)
     w = workloads.make(shape=shape, device="cuda", seed=8)
     q = w.q.to(q_dtype)
+    one = cascade._one_sequence(batch * queries * q_heads // 8, pages * 16, 8, q_dtype, w.k_cache.dtype)
+    assert one == (pages in (114, 200, 384, 249))
     want, _ = oracle_of(w, q)
     got = cascade_decode_attention(q, *w.args()[1:], **w.kwargs(), prefix_pages=pages, out_dtype=q_dtype,
                                    context_lens_host=w.lengths)

@@ -103,10 +103,13 @@ def test_norm_quant_needs_gpu_tensors():
 
 def test_cascade_prefix_as_one_sequence():
     bf, f8 = torch.bfloat16, torch.float8_e4m3fn
-    assert cascade._one_sequence(32, 2048, bf, bf) and not cascade._one_sequence(32, 2047, bf, bf)
-    assert cascade._one_sequence(512, 2048, torch.float16, f8) and not cascade._one_sequence(512, 2047, bf, f8)
-    assert not cascade._one_sequence(512, 8192, torch.float32, bf)  # an f32 q keeps float32 products
-    assert not cascade._one_sequence(16, 1 << 20, bf, f8)
+    one = cascade._one_sequence
+    assert one(32, 2048, 8, bf, bf) and not one(32, 2047, 8, bf, bf)
+    assert one(32, 16384, 1, bf, bf) and not one(32, 16383, 1, bf, bf)  # the work of all KV heads counts
+    assert one(512, 6144, 8, torch.float16, f8) and not one(512, 6143, 8, bf, f8)
+    assert one(512, 4096, 8, bf, torch.int8) and not one(512, 4095, 8, bf, torch.int8)
+    assert not one(512, 8192, 8, torch.float32, bf)  # an f32 q keeps float32 products
+    assert not one(16, 1 << 20, 8, bf, f8)
 
 
 def test_cascade_rows_per_pass():
