@@ -253,3 +253,22 @@ def test_rows_values_that_are_not_finite_reach_only_the_rows_that_see_them(fmt, 
     assert np.array_equal(np.isfinite(got), fin)
     assert np.array_equal(got[~fin], want[~fin], equal_nan=True)
     assert np.abs(got[fin] - want[fin]).max() <= 2.0**-14 * np.abs(want[fin]).max()
+
+
+@pytest.mark.parametrize("fmt,scales", [("fp8", "token"), ("bf16", None)])
+@pytest.mark.parametrize("nq,tile", [(20, 32), (40, 64), (128, 128), (200, 256)])
+def test_rows_at_the_longest_tile_line(fmt, scales, nq, tile):
+    """2048 sequences of one tile each fill the line in LDS (4096 entries) beside the chunk buffers of every tile size: a
+    launch that asked for too much would be refused. The first, some middle and the last sequences against the oracle."""
+    from bpt_amd import decode_plan, paged_decode_attention
+
+    g = torch.Generator().manual_seed(nq)
+    lengths = torch.randint(0, 2 * nq, (2048,), generator=g).tolist()
+    c = make_case(fmt, lengths, hq=1, hkv=1, nq=nq, scales=scales, seed=nq)
+    args = (c["q"], c["k"], c["v"], c["table"], c["lens"], c["ks"], c["vs"])
+    plan = decode_plan(*args, scale=0.0883883, max_context=512)
+    assert plan[1] == 128 and plan[2] == -(-2 * plan[0] * tile * 129 * 4 // 256) * 256
+    got = paged_decode_attention(*args, scale=0.0883883, max_context=512)
+    for at in (slice(0, 4), slice(1023, 1026), slice(2045, 2048)):
+        part = dict(c, q=c["q"][at], table=c["table"][at], lens=c["lens"][at])
+        check(got[at], run_case(part)[1], f"{fmt} {nq} queries, sequences {at}")
