@@ -128,14 +128,14 @@ def quantize_args(k: torch.Tensor, v: torch.Tensor, kv: Any, start: int) -> Any:
         raise ValueError("the cache's batch and KV heads must match")
     if not (start >= 0 and start % kv.group == 0 and start + n <= kv.k_codes.shape[2]):
         raise ValueError(f"tokens {start} .. {start + n} must start on a key group and fit the cache")
-    if not (kv.bits in (4, 8)):
+    if kv.bits not in (4, 8):
         raise ValueError(f"bits must be 4, 8 or 16, got {kv.bits}")
-    if not (n % kv.group == 0):
+    if n % kv.group != 0:
         raise ValueError(f"{n} tokens are not a whole number of groups of {kv.group}")
     if not (k.dtype in _Q_CODES and k.stride(-1) == 1):
         raise ValueError("k and v must be bf16, f16 or f32 with contiguous channels")
     dev = k.device
-    if not (dev.type == "cuda"):
+    if dev.type != "cuda":
         raise ValueError("quantize_kv runs on a GPU: k must be a cuda tensor")
     kc = kv.k_codes[:, :, start:start + n]
     vc = kv.v_codes[:, :, start:start + n]
@@ -146,14 +146,14 @@ def quantize_args(k: torch.Tensor, v: torch.Tensor, kv: Any, start: int) -> Any:
         raise ValueError("codes: uint8, shared layout")
     if not (kc.shape[3] * (2 if kv.bits == 4 else 1) == d):
         raise ValueError(f"codes hold {kc.shape[3]} bytes per token, k has D={d}")
-    if not (all(t.dtype == torch.float16 for t in (ks, kz, vs, vz))):
+    if not all(t.dtype == torch.float16 for t in (ks, kz, vs, vz)):
         raise ValueError("grids must be float16")
     if not (ks.stride() == kz.stride() and ks.stride(-1) == 1):
         raise ValueError("key grids: shared layout, contiguous channels")
     if not (vs.stride() == vz.stride() and vs.stride(-1) == 1):
         raise ValueError("value grids: shared layout, unit token stride")
     for t in (v, kc, vc, ks, kz, vs, vz):
-        if not (t.device == dev):
+        if t.device != dev:
             raise ValueError(f"every tensor must be on {dev}")
     a = _lib.KiviQuantArgs()
     a.struct_size = ctypes.sizeof(_lib.KiviQuantArgs)
@@ -200,7 +200,7 @@ def _launch(q, kv, lengths, scale, split, n_splits, out, lse, tail=None) -> None
     kc, vc = kv.k_codes, kv.v_codes
     if not (kc.dim() == 4 and kc.shape == vc.shape):
         raise ValueError("k_codes and v_codes must be [B, Hkv, T, E] of one shape")
-    if not (kc.shape[0] == b):
+    if kc.shape[0] != b:
         raise ValueError(f"the cache holds {kc.shape[0]} sequences, q {b}")
     hkv, t_max = kc.shape[1], kc.shape[2]
     quant = fmt in (KIVI_INT4, KIVI_INT8)
@@ -212,18 +212,18 @@ def _launch(q, kv, lengths, scale, split, n_splits, out, lse, tail=None) -> None
     else:
         if not (vc.dtype == kc.dtype and kc.shape[3] == d):
             raise ValueError("bits-16 keys and values must share q's head dim and a dtype")
-    if not (q.dtype in _Q_CODES):
+    if q.dtype not in _Q_CODES:
         raise ValueError(f"q must be bfloat16, float16 or float32, got {q.dtype}")
     if not (q.stride(-1) == 1 and kc.stride(-1) == 1 and vc.stride() == kc.stride()):
         raise ValueError("channels must be contiguous")
     if not (lengths.dtype == torch.int32 and tuple(lengths.shape) == (b,) and lengths.is_contiguous()):
         raise ValueError(f"lengths must be int32 [{b}]")
     dev = q.device
-    if not (dev.type == "cuda"):
+    if dev.type != "cuda":
         raise ValueError("decode_attention runs on a GPU: q must be a cuda tensor")
     grids = (kv.k_scale, kv.k_zero, kv.v_scale, kv.v_zero) if quant else ()
     for t in (kc, vc, lengths, *grids):
-        if not (t.device == dev):
+        if t.device != dev:
             raise ValueError(f"every tensor must be on {dev}")
 
     a = _lib.KiviArgs()
@@ -239,7 +239,7 @@ def _launch(q, kv, lengths, scale, split, n_splits, out, lse, tail=None) -> None
     if quant:
         ks, kz, vs, vz = grids
         for name, g in (("k_scale", ks), ("k_zero", kz), ("v_scale", vs), ("v_zero", vz)):
-            if not (g.dtype == torch.float16):
+            if g.dtype != torch.float16:
                 raise ValueError(f"{name} must be float16, got {g.dtype}")
         if not (ks.dim() == 4 and ks.shape == kz.shape and tuple(ks.shape[:2]) == (b, hkv) and ks.shape[3] == d):
             raise ValueError(f"k_scale / k_zero must be [{b}, {hkv}, groups, {d}]")
