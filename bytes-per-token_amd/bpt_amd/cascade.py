@@ -12,9 +12,9 @@ tile of up to 256 of them where the group's rows and the prefix are many (_one_s
    result is merged with its prefix partial as kernels/reference.py:205-211 merges split partials, so the
    output is the attention over the whole context.
 
-Both passes are calls of the library's paged decode (one per group and one for the suffixes; a call is one launch, or two
-where a large call's split tiles are combined by a second one); the merge happens in the suffix pass's final write. The result equals `paged_decode_attention` on the same
-inputs up to float32 rounding.
+Both passes are calls of the library's paged decode, one per group and one for the suffixes (a call is one
+launch, or two where a large call's split tiles are combined by a second one); the merge happens in the suffix
+pass's final write. The result equals `paged_decode_attention` on the same inputs up to float32 rounding.
 
 Requirements: every sequence of a group holds the group's prefix in its first `prefix_pages` block-table
 entries (the same physical pages), all groups share one prefix length, and every query sits at or after
@@ -82,15 +82,15 @@ def cascade_decode_attention(
     q4 = q[:, None] if squeeze else q
     b, nq, hq, d = q4.shape
     hkv, page = k_cache.shape[2], k_cache.shape[1]
-    if not (hq % hkv == 0):
+    if hq % hkv != 0:
         raise ValueError(f"{hq} query heads are not a multiple of {hkv} KV heads")
     heads_per_kv = hq // hkv
-    if not (prefix_pages >= 1):
+    if prefix_pages < 1:
         raise ValueError("prefix_pages must be at least 1 (use paged_decode_attention without a prefix)")
     if not (block_table.dim() == 2 and block_table.shape[1] >= prefix_pages):
         raise ValueError(f"block_table must hold at least the {prefix_pages} prefix pages")
     prefix = prefix_pages * page
-    if not (max_context >= prefix):
+    if max_context < prefix:
         raise ValueError(f"max_context {max_context} is shorter than the {prefix}-token prefix")
     groups = [(0, b)] if groups is None else [(int(s), int(e)) for s, e in groups]
     at = 0
@@ -98,11 +98,11 @@ def cascade_decode_attention(
         if not (s == at and e > s):
             raise ValueError("groups must be consecutive, non-empty [start, end) ranges covering the batch")
         at = e
-    if not (at == b):
+    if at != b:
         raise ValueError("groups must cover the whole batch")
     if context_lens_host is not None:
         short = [i for i, n in enumerate(context_lens_host) if n < prefix + nq - 1]
-        if not (not short):
+        if short:
             raise ValueError(f"sequences {short[:8]} end inside the shared prefix: their queries would see all of it")
     dev = q4.device
     q4c = q4 if q4.stride(0) == nq * q4.stride(1) and q4.stride(1) == hq * q4.stride(2) and q4.stride(2) == d else q4.contiguous()

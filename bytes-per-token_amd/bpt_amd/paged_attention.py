@@ -66,7 +66,7 @@ def _scale_layout(k_scale, v_scale, kv_code: int, pool_shape) -> tuple[int, tupl
     if not (k_scale is not None and v_scale is not None):
         raise ValueError("k_scale and v_scale are required for a quantized cache")
     for s in (k_scale, v_scale):
-        if not (s.dtype == torch.float32):
+        if s.dtype != torch.float32:
             raise ValueError(f"scales must be float32, got {s.dtype}")
     nb, p, hkv, _ = pool_shape
     if k_scale.dim() == 1:
@@ -77,7 +77,7 @@ def _scale_layout(k_scale, v_scale, kv_code: int, pool_shape) -> tuple[int, tupl
         return SCALE_PER_HEAD, (0, 0, 0)
     if not (tuple(k_scale.shape) == (nb, p, hkv) and tuple(v_scale.shape) == (nb, p, hkv)):
         raise ValueError(f"per-token-head scales must be [{nb}, {p}, {hkv}] like the pools")
-    if not (k_scale.stride() == v_scale.stride()):
+    if k_scale.stride() != v_scale.stride():
         raise ValueError("k_scale and v_scale must share strides")
     return SCALE_PER_TOKEN_HEAD, tuple(k_scale.stride())
 
@@ -85,37 +85,37 @@ def _scale_layout(k_scale, v_scale, kv_code: int, pool_shape) -> tuple[int, tupl
 def _decode_args(
     q, k_cache, v_cache, block_table, context_lens, k_scale, v_scale, scale, max_context, num_splits, out_dtype
 ) -> tuple[_lib.DecodeArgs, tuple[int, int, int, int]]:
-    if not (q.dim() == 4):
+    if q.dim() != 4:
         raise ValueError(f"q must be [B, Q, Hq, D], got {tuple(q.shape)}")
     b, nq, hq, d = q.shape
-    if not (q.dtype in _FLOAT_CODES):
+    if q.dtype not in _FLOAT_CODES:
         raise ValueError(f"q must be bf16, f16 or f32, got {q.dtype}")
-    if not (q.stride(-1) == 1):
+    if q.stride(-1) != 1:
         raise ValueError("q's channel dimension must be contiguous")
     if not (k_cache.dim() == 4 and k_cache.shape == v_cache.shape):
         raise ValueError("k_cache and v_cache must be [NB, P, Hkv, D]")
-    if not (k_cache.dtype == v_cache.dtype):
+    if k_cache.dtype != v_cache.dtype:
         raise ValueError("k_cache and v_cache must share a dtype")
-    if not (k_cache.stride() == v_cache.stride()):
+    if k_cache.stride() != v_cache.stride():
         raise ValueError("k_cache and v_cache must share strides")
-    if not (k_cache.stride(-1) == 1):
+    if k_cache.stride(-1) != 1:
         raise ValueError("the caches' channel dimension must be contiguous")
     kv_code = kv_dtype_code(k_cache.dtype)
     nb, page, hkv, dk = k_cache.shape
-    if not (dk == d):
+    if dk != d:
         raise ValueError(f"q head_dim {d} != cache head_dim {dk}")
     if not (block_table.dim() == 2 and block_table.shape[0] == b):
         raise ValueError(f"block_table must be [{b}, max_blocks]")
-    if not (block_table.dtype in _INDEX_CODES):
+    if block_table.dtype not in _INDEX_CODES:
         raise ValueError("block_table must be int32 or int64")
-    if not (block_table.stride(1) == 1):
+    if block_table.stride(1) != 1:
         raise ValueError("block_table rows must be contiguous")
     if context_lens is not None:
         if not (context_lens.dim() == 1 and context_lens.shape[0] == b):
             raise ValueError(f"context_lens must be [{b}]")
         if not (context_lens.dtype == torch.int32 and context_lens.is_contiguous()):
             raise ValueError("context_lens must be contiguous int32")
-    if not (out_dtype in _FLOAT_CODES):
+    if out_dtype not in _FLOAT_CODES:
         raise ValueError(f"out dtype must be bf16, f16 or f32, got {out_dtype}")
     scale_kind, sc_strides = _scale_layout(k_scale, v_scale, kv_code, k_cache.shape)
 
@@ -227,7 +227,8 @@ def paged_decode_attention(
                   scale * q.k over the tokens it saw (natural log, -inf for none): with `out` in float32 it is
                   the partial that kernels/reference.py:205-211 merges
 
-    Returns out [B, Q, Hq, D] (or [B, Hq, D]) in `out_dtype` (bf16 by default). One kernel launch.
+    Returns out [B, Q, Hq, D] (or [B, Hq, D]) in `out_dtype` (bf16 by default). One kernel launch, or two where a large call
+    with more than 16 query rows per KV head (Q x Hq / Hkv) combines its partials in a second.
     """
     squeeze = q.dim() == 3
     q4 = q[:, None] if squeeze else q
@@ -246,7 +247,7 @@ def paged_decode_attention(
         out4 = torch.empty((b, nq, hq, d), dtype=out_dtype, device=dev)
     else:
         out4 = out[:, None] if out.dim() == 3 else out
-        if not (tuple(out4.shape) == (b, nq, hq, d)):
+        if tuple(out4.shape) != (b, nq, hq, d):
             raise ValueError(f"out must be [{b}, {nq}, {hq}, {d}]")
         if not (out4.stride(-1) == 1 and out4.device == dev):
             raise ValueError("out must be a cuda tensor with contiguous channels")
@@ -256,7 +257,7 @@ def paged_decode_attention(
         if not (lse.dtype == torch.float32 and lse.is_contiguous() and lse.numel() == b * nq * hq and lse.device == dev):
             raise ValueError(f"lse must be a contiguous float32 tensor of {b} x {nq} x {hq} on q's device")
         a.lse_out = lse.data_ptr()
-    if _cascade is not None:  # the cascade's two launches (cascade.py): flags, length offset, partial to merge
+    if _cascade is not None:  # the cascade's passes (cascade.py): flags, length offset, partial to merge
         a.flags = _cascade.get("flags", 0)
         a.len_offset = _cascade.get("len_offset", 0)
         merge = _cascade.get("merge")
@@ -327,7 +328,7 @@ def _append_args(k, v, k_cache, v_cache, k_scale, v_scale, write_blocks, write_o
         raise ValueError("caches must match")
     if not (k_cache.shape[2] == hkv and k_cache.shape[3] == d):
         raise ValueError("cache heads/head_dim must match the rows")
-    if not (k_cache.stride(-1) == 1):
+    if k_cache.stride(-1) != 1:
         raise ValueError("the caches' channel dimension must be contiguous")
     kv_code = kv_dtype_code(k_cache.dtype)
     scale_kind, sc_strides = _scale_layout(k_scale, v_scale, kv_code, k_cache.shape)
@@ -335,14 +336,14 @@ def _append_args(k, v, k_cache, v_cache, k_scale, v_scale, write_blocks, write_o
         raise ValueError(f"write slots must be [{b}, {nq}]")
     if not (write_blocks.dtype == write_offsets.dtype and write_blocks.dtype in _INDEX_CODES):
         raise ValueError("slots: int32/int64")
-    if not (write_blocks.stride() == write_offsets.stride()):
+    if write_blocks.stride() != write_offsets.stride():
         raise ValueError("write_blocks and write_offsets must share strides")
     dev = k.device
-    if not (dev.type == "cuda"):
+    if dev.type != "cuda":
         raise ValueError("quantize_append runs on a GPU: k must be a cuda tensor")
     for name, t in (("v", v), ("k_cache", k_cache), ("v_cache", v_cache), ("write_blocks", write_blocks),
                     ("write_offsets", write_offsets), ("k_scale", k_scale), ("v_scale", v_scale)):
-        if not (t is None or t.device == dev):
+        if t is not None and t.device != dev:
             raise ValueError(f"{name} is not on {dev}")
 
     n_sb, n_sq, n_sh, _ = k.stride()
@@ -387,7 +388,7 @@ def paged_append_decode(
     same results.
     """
     a, dev = _append_args(k, v, k_cache, v_cache, k_scale, v_scale, write_blocks, write_offsets)
-    if not (q.device == dev):
+    if q.device != dev:
         raise ValueError(f"q is on {q.device}, the new rows on {dev}")
     return paged_decode_attention(q, k_cache, v_cache, block_table, context_lens, k_scale, v_scale, scale=scale,
                                   max_context=max_context, num_splits=num_splits, out=out, out_dtype=out_dtype,
@@ -428,7 +429,7 @@ def paged_prepare(
         raise ValueError(f"block_table: [{b}, n_blocks]")
     dev = positions.device
     for name, t in (("table", table), ("reserved", reserved), ("slots", slots), ("block_table", block_table)):
-        if not (t.device == dev):
+        if t.device != dev:
             raise ValueError(f"{name} is not on {dev}")
     a = _lib.PrepareArgs()
     a.struct_size = ctypes.sizeof(_lib.PrepareArgs)

@@ -146,9 +146,9 @@ constexpr int kMfmaChunk = 32;
 // Many-row attention (decode_rows.h): chunks of kRowsChunk tokens, tiles of 32, 64, 128 or 256 rows. A 256-row tile
 // decodes each chunk once for twice the rows of a 128-row one and its waves share nothing, but its pieces are twice as
 // large: it is taken from kRowsWideChunks (tile, chunk) units on, eight per CU. Measured, 256 against 128 rows (us):
-// FP8 2048 + 2048 tokens, 16 heads (4096 units) 121 : 138; INT8 512 + 8192, 32 heads (4352) 165 : 191; FP8 150 + 12000,
-// 64 heads (3800) 132 : 152; FP8 3 x (40 + 2000), 32 heads (384) 35 : 35; FP8 100 + 1000, 16 heads (72) 26 : 23; BF16
-// 4 x 300, 32 heads (480) 51 : 47.
+// 2048 + 2048 tokens, 16 heads (4096 units) FP8 118 : 129, INT8 143 : 150, BF16 138 : 148; 512 + 8192, 32 heads (4352)
+// INT8 177 : 195; 150 + 12000, 64 heads (3800) FP8 122 : 142, INT8 155 : 174, BF16 153 : 181; FP8 3 x (40 + 2000), 32 heads
+// (384) 35 : 35; BF16 4 x 300, 32 heads (480) 51 : 47.
 constexpr int kRowsChunk = 128;
 constexpr int64_t kRowsWideChunks = 8 * kComputeUnits;
 // Rows of a tile below that: the fewest that hold a KV head's rows, or that still leave no more than one (tile, chunk) unit

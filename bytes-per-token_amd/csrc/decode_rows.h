@@ -4,7 +4,8 @@
 // A tile is BM consecutive rows (row r = query r / G, head h G + r % G) of one (sequence, KV head); it walks the
 // chunks of kRowsChunk tokens that its last row sees (causal: later tokens are never read for it). The tiles' chunks
 // are laid end to end on a line that the workgroups cut into equal ranges, as in the decode kernels (decode_common.h):
-// a tile held by one workgroup is written directly, the others go through partials that the last arriver combines.
+// a tile held by one workgroup is written directly, the others go through partials that the last arriver combines or,
+// where they are large, a second launch (rows_combine_kernel).
 //
 // One workgroup = NW waves = WM row blocks of 32 rows x WN token groups. Per chunk:
 //  * all waves load the chunk's K and V codes (whole 16-token groups, one page lookup each), decode them once to
@@ -20,11 +21,11 @@
 // 32 heads 154 us against 172, but drops bits that the vector kernel keeps, and scales past 2^64.)
 //
 // What bounds it: with many chunks the matrix cores (FP8: three products where two would do, for the weights' second
-// part) and the vector units behind them (256-row tiles, 2048 rows x 8 heads over 4096 tokens: 37 % and 52 % of the
-// cycles, and leaving out the second part, the exponentials or the decoding saves 15, 5 and 5 of 122 us); with few the
-// first loads and the partials. Measured against the vector kernel's 4-row groups, which decode every chunk rows / 4
-// times (8 KV heads, us): FP8 prompt chunks of 2048 over 2048 cached tokens, 16 heads 1885 -> 121; verifies of 5
-// queries, 32 heads, 16 sequences of 1024..3072 tokens 113 -> 34.
+// part) and the vector units, mostly in turn (256-row tiles, 2048 queries x 16 heads over 4096 tokens: busy for 42 % and
+// 51 % of the cycles); with few the first loads and the partials. Kernel times against the vector kernel's 4-row groups,
+// which decode every chunk rows / 4 times (8 KV heads, us): FP8 prompt chunks of 2048 over 2048 cached tokens, 16 heads
+// 1885 -> 129 (114 and 15 in the combine's launch); verifies of 5 queries, 32 heads, 16 sequences of 1024..3072 tokens
+// 113 -> 34.
 //
 // LDS layouts (16-byte units; both spread the 8 lanes that one LDS cycle serves over all banks):
 //  * K: token row of 16 units, unit u at u ^ (token % 8) ^ (u / 8). Operand reads take one unit of 8 consecutive
@@ -708,9 +709,9 @@ __device__ __forceinline__ void rows_combine(const DecodeParams& p, int b, int h
 }
 
 // The combine as a launch of its own (DecodeParams::two_pass): the workgroups take strips of kCombineRows rows of the
-// tiles in turn, the pieces in the slots of rows_combine. The last arriver of a tile is one CU, which reads some 50 GB/s
-// past the L2s, so 33 pieces of 128 rows (2 MiB) took it about 25 us. Spread over the chip they take 5.5 us: a call whose
-// tiles have much to combine pays a second launch instead (rows_two_pass), and its pieces are plain stores.
+// tiles in turn, the pieces in the slots of rows_combine. The last arriver of a tile is one CU: 33 pieces of 128 rows
+// (64 KiB each) took it about 25 us, some 85 GB/s. Spread over the chip they take 5.5 us: a call whose tiles have much to
+// combine pays a second launch instead (rows_two_pass), and its pieces are plain stores.
 constexpr int kCombineRows = 8, kCombineWaves = 4, kCombineGrid = 4 * kComputeUnits;
 template <int BM>
 __global__ __launch_bounds__(kCombineWaves * 64) void rows_combine_kernel(const DecodeParams p) {

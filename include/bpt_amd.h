@@ -86,8 +86,8 @@ typedef enum { BPT_IDX_I32 = 0, BPT_IDX_I64 = 1 } bpt_index_dtype;
  * above max_blocks_per_seq * page_size, are truncated to that bound. Page ids are clamped into
  * [0, num_blocks). batch is at most 4096.
  *
- * Split-K: each (sequence, KV head) is cut into partitions whose log-sum-exp partials are combined exactly
- * inside the same launch. num_splits = 0 balances the whole batch over the launched workgroups (ragged
+ * Split-K: each (sequence, KV head) is cut into partitions whose log-sum-exp partials are combined exactly, inside the
+ * same launch or, where a call with more than 16 query rows per KV head has large ones, by a second launch. num_splits = 0 balances the whole batch over the launched workgroups (ragged
  * lengths included); num_splits = S > 0 cuts a max_context-long sequence into S partitions (shorter ones
  * into proportionally fewer).
  *
@@ -365,7 +365,8 @@ typedef struct {
  * bytes. Touches no GPU. */
 int bpt_decode_plan(bpt_decode_args* args, size_t* workspace_bytes, size_t* counters_bytes);
 
-/* Paged decode attention: one kernel launch, split-K partials combined in the same launch. */
+/* Paged decode attention: one kernel launch, or two (the split-K partials of large calls with more than 16 query rows per
+ * KV head are combined by the second). */
 int bpt_paged_decode(const bpt_decode_args* args, void* stream);
 
 /* bpt_paged_decode with no caller workspace: the split-K partials and arrival counters live in a device-
