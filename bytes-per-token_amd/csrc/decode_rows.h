@@ -378,11 +378,14 @@ __device__ __forceinline__ f32x16 rows_scores(const u32x4 (&ka)[8], const u32x4 
   f32x16 s;
 #pragma unroll
   for (int i = 0; i < 16; ++i) s[i] = 0.0f;
+  // An f16 q's remainders go first, while the sum is small: they then cost it no rounding (float32 outputs 5.3e-7 from 64
+  // bits at 512 + 2048 tokens, 16 heads, and 6.9e-7 with each after its high part; 512 + 8192, 32 heads 199 -> 203 us).
+  if constexpr (C::kQSplit) {
 #pragma unroll
-  for (int k = 0; k < 8; ++k) {
-    s = rows_mfma_k<C>(ka[k], qb[k], s);
-    if constexpr (C::kQSplit) s = rows_mfma_k<C>(ka[k], qb[8 + k], s);
+    for (int k = 0; k < 8; ++k) s = rows_mfma_k<C>(ka[k], qb[8 + k], s);
   }
+#pragma unroll
+  for (int k = 0; k < 8; ++k) s = rows_mfma_k<C>(ka[k], qb[k], s);
   return s;
 }
 // The V operands (A) of the 16 tokens from t0 on: one per 32 channels.
